@@ -195,7 +195,7 @@ int check_gemm(const frisk_gemm_desc* d, const char* fn, bool ptrs, frisk::GemmA
   // transposed) whole 16 B pieces of K; the epilogue stores 16 B per lane
   // into C rows.  Their buffer loads take 32-bit offsets from one tile
   // origin: a K-major operand reaches (rows - 1) pitches plus K, an MN-major
-  // one (K - 1) pitches plus a tile row; beyond 2^31 - 1 bytes the generic
+  // one (K - 1) pitches plus a tile row; beyond 2^31 - 1 bytes the any-alignment
   // kernel (64-bit indexing) runs instead.
   const int ies = esize(d->a_type), oes = esize(d->c_type);
   const bool a_kmajor = !g.trans_a, b_kmajor = g.trans_b;
@@ -295,7 +295,7 @@ int launch_gemm(const frisk::GemmArgs& g, GemmRoute route, void* ws, int64_t ws_
   } else if (route == GemmRoute::Mfma) {
     e = frisk::gemm_mfma(g, (hipStream_t)stream, ws, ws_bytes);
   } else {
-    e = frisk::gemm_generic_any(g, (hipStream_t)stream);
+    e = frisk::gemm_any(g, (hipStream_t)stream, ws, ws_bytes);
   }
   if (e != hipSuccess) return fail(FRISK_EHIP, "%s launch: %s", fn, hipGetErrorString(e));
   return FRISK_OK;
@@ -337,10 +337,12 @@ int frisk_gemm_plan(const frisk_gemm_desc* d, char* buf, int64_t len) {
   int n = 0;
   if (L.kernel == frisk::plan::Kernel::Generic) {
     n = snprintf(buf, (size_t)len,
-                 "{\"kernel\": \"gemm_generic\", \"tile_m\": 64, \"tile_n\": 64, \"atom\": \"fma\", "
-                 "\"a_major\": \"%s\", \"b_major\": \"%s\", \"slices\": 1, \"slice_sum\": \"none\", "
-                 "\"workspace_bytes\": 0}",
-                 a_major, b_major);
+                 "{\"kernel\": \"gemm_generic\", \"tile_m\": %d, \"tile_n\": %d, \"atom\": \"%s\", "
+                 "\"waves\": [2, 2], \"stage_bytes\": %d, \"a_major\": \"%s\", \"b_major\": \"%s\", "
+                 "\"slices\": %d, \"slice_sum\": \"%s\", \"workspace_bytes\": %lld}",
+                 L.tile_m, L.tile_n, mfma_atom(g.in == frisk::Elt::E4M3 ? frisk::Elt::F16 : g.in),
+                 L.stage_bytes, a_major, b_major, L.slices,
+                 slice_sum, (long long)L.workspace_bytes);
   } else if (L.kernel == frisk::plan::Kernel::Skinny) {
     n = snprintf(buf, (size_t)len,
                  "{\"kernel\": \"gemm_skinny\", \"tile_m\": %d, \"tile_n\": %d, "
@@ -387,7 +389,10 @@ int frisk_gemm(const frisk_gemm_desc* d, void* stream) {
   int64_t ws_bytes = 0;
   if (d->workspace) {
     const int64_t need = gemm_workspace(g, route);
-    if (need > 0) {
+    const bool fits = d->workspace_bytes >= need && (uintptr_t)d->workspace % 16 == 0;
+    // The any-alignment kernel runs unsplit where the others reject a short
+    // or misaligned workspace: its callers may pass one sized for another GEMM.
+    if (need > 0 && (fits || route != GemmRoute::Generic)) {
       if (d->workspace_bytes < need)
         return fail(FRISK_EINVAL, "frisk_gemm: workspace of %lld bytes, this GEMM takes %lld",
                     (long long)d->workspace_bytes, (long long)need);

@@ -333,7 +333,7 @@ static hipError_t launch_128_split_k(const GemmArgs& g, int slices, int64_t kb_s
                        (int64_t)g.m * g.n * 4, SplitTree{});
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    return gemm_splitk_sum((const float*)ws, slices, g, stream);
+    return gemm_splitk_sum(ws, slices, g.n, g, stream);
   }
 }
 

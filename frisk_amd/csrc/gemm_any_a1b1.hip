@@ -1,0 +1,8 @@
+// The any-alignment MFMA GEMM (gemm_any.h) for trans_a = 1, trans_b = 1:
+// A stored [K, M], B stored [N, K].
+#include "gemm_any.h"
+
+namespace frisk {
+template hipError_t gemm_any_layout<true, false>(const GemmArgs&, const plan::SplitPlan&, void*,
+                                             hipStream_t);
+}  // namespace frisk

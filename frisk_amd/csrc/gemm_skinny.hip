@@ -188,26 +188,37 @@ __global__ __launch_bounds__(64 * kSkinnyWaves) void gemm_skinny_kernel(
 #endif  // __HIP_DEVICE_COMPILE__
 }
 
-// C[row, 4c .. 4c+3] (+)= sum over slices z = 0, 1, ... of
-// partial[z][row][4c .. 4c+3], added in slice order.  N is a multiple of 4.
+// C[row, 4c .. 4c+3] (+)= scale * (sum over slices z = 0, 1, ... of
+// partial[z][row][4c .. 4c+3], added in slice order).  Partial rows are
+// `pitch` elements, a multiple of 4; columns past N are not stored.  An i32
+// output sums i32 partials.
 template <Elt OUT>
-__global__ __launch_bounds__(256) void gemm_splitk_sum_kernel(const float* __restrict__ partial,
-                                                              int slices, int M, int N,
+__global__ __launch_bounds__(256) void gemm_splitk_sum_kernel(const void* __restrict__ partial,
+                                                              int slices, int M, int N, int pitch,
                                                               void* __restrict__ C, int64_t ldc,
-                                                              int accumulate) {
-  const int64_t quads = (int64_t)N / 4;
+                                                              float scale, int accumulate) {
+  using V = typename std::conditional<OUT == Elt::I32, i32x4, f32x4>::type;
+  const int64_t quads = (int64_t)pitch / 4;
   const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (idx >= (int64_t)M * quads) return;
   const int row = (int)(idx / quads), col = (int)(idx % quads) * 4;
-  f32x4 sum = *(const f32x4*)(partial + (int64_t)row * N + col);
+  const char* p = (const char*)partial + ((int64_t)row * pitch + col) * 4;
+  const int64_t slice_bytes = (int64_t)M * pitch * 4;
+  V sum = *(const V*)p;
 #pragma unroll 8
-  for (int z = 1; z < slices; ++z) sum += *(const f32x4*)(partial + ((int64_t)z * M + row) * N + col);
+  for (int z = 1; z < slices; ++z) sum += *(const V*)(p + z * slice_bytes);
   const int64_t o = (int64_t)row * ldc + col;
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
-    float v = sum[e];
-    if (accumulate) v += load_as_f32<OUT>(C, o + e);
-    store_from_f32<OUT>(C, o + e, v);
+    if (col + e >= N) break;
+    if constexpr (OUT == Elt::I32) {
+      int32_t* c = (int32_t*)C + o + e;
+      *c = accumulate ? *c + sum[e] : sum[e];
+    } else {
+      float v = sum[e] * scale;
+      if (accumulate) v += load_as_f32<OUT>(C, o + e);
+      store_from_f32<OUT>(C, o + e, v);
+    }
   }
 }
 
@@ -226,7 +237,7 @@ hipError_t launch_skinny(const GemmArgs& g, const SkinnyPlan& p, float* partial,
                      partial);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || !partial) return e;
-  return gemm_splitk_sum(partial, p.slices, g, stream);
+  return gemm_splitk_sum(partial, p.slices, g.n, g, stream);
 }
 
 template <Elt IN, Elt OUT, int TN>
@@ -250,25 +261,24 @@ hipError_t skinny_by_n(const GemmArgs& g, const SkinnyPlan& p, float* partial, h
 
 }  // namespace
 
-hipError_t gemm_splitk_sum(const float* partial, int slices, const GemmArgs& g, hipStream_t s) {
-  const int64_t threads = g.m * (g.n / 4);
+hipError_t gemm_splitk_sum(const void* partial, int slices, int64_t pitch, const GemmArgs& g,
+                           hipStream_t s) {
+  const int64_t threads = g.m * (pitch / 4);
   const dim3 grid((unsigned)((threads + 255) / 256));
+#define FRISK_SUM(O)                                                                              \
+  case Elt::O:                                                                                    \
+    hipLaunchKernelGGL((gemm_splitk_sum_kernel<Elt::O>), grid, dim3(256), 0, s, partial, slices,  \
+                       (int)g.m, (int)g.n, (int)pitch, g.c, g.ldc, g.scale, g.accumulate);        \
+    break;
   switch (g.out) {
-    case Elt::BF16:
-      hipLaunchKernelGGL((gemm_splitk_sum_kernel<Elt::BF16>), grid, dim3(256), 0, s, partial,
-                         slices, (int)g.m, (int)g.n, g.c, g.ldc, g.accumulate);
-      break;
-    case Elt::F16:
-      hipLaunchKernelGGL((gemm_splitk_sum_kernel<Elt::F16>), grid, dim3(256), 0, s, partial,
-                         slices, (int)g.m, (int)g.n, g.c, g.ldc, g.accumulate);
-      break;
-    case Elt::F32:
-      hipLaunchKernelGGL((gemm_splitk_sum_kernel<Elt::F32>), grid, dim3(256), 0, s, partial,
-                         slices, (int)g.m, (int)g.n, g.c, g.ldc, g.accumulate);
-      break;
+    FRISK_SUM(BF16)
+    FRISK_SUM(F16)
+    FRISK_SUM(F32)
+    FRISK_SUM(I32)
     default:
       return hipErrorInvalidValue;
   }
+#undef FRISK_SUM
   return hipGetLastError();
 }
 

@@ -50,7 +50,10 @@
 //    swz(r) = (r & 7) << 1 gives each row its own 32 B pair of chunks.
 //  * MN-major 8-bit, 128 B rows: two rows share a window (r & 1 picks the
 //    half); swz(r) = ((r >> 1) & 3) << 1 separates the four pairs of rows.
-//  * MN-major 32-bit (rows of 512 or 1024 B): a ds_read_b32 has lanes 0-31
+//  * MN-major rows of a 64-column tile: 16-bit, 128 B, where rows e and e + 2
+//    share a half window, swz(r) = ((r >> 1) & 1) << 2; 8-bit, 64 B, where
+//    rows e and e + 4 share a quarter, swz(r) = ((r >> 2) & 1) << 1.
+//  * MN-major 32-bit (rows of 256 to 1024 B): a ds_read_b32 has lanes 0-31
 //    on 128 contiguous bytes of k-row e and lanes 32-63 on k-row 4 + e;
 //    swz(r) = ((r >> 2) & 1) << 3 moves the second row 128 B over, onto the
 //    other 32 banks.
@@ -80,7 +83,8 @@ struct OpTile {
   static constexpr int kLaneK = Op::kBytes / kGroups / kEsz;  // k per lane per MFMA
   static constexpr int kReadsPerChunk = MN ? (kEsz == 4 ? 4 : 2) : 1;  // LDS reads per 16 B
   static_assert(kRows * kRB == kBytes && kRowsPerBlock >= 1, "tile geometry");
-  static_assert(!MN || kRB >= 128, "MN-major rows of at least 128 B");
+  static_assert(!MN || kRB >= 64, "MN-major rows of at least 64 B");
+  static_assert(ATOM == 32 || (BT >= 128 && KR <= 128), "16x16 atoms on tiles of 128 rows");
   static_assert(ATOM == 32 || ATOM == 16, "MFMA atom");
   static_assert(kEsz != 4 || ATOM == 32, "32-bit operands on 32x32 atoms");
   static_assert(KR % Op::kBytes == 0, "whole MFMA k-steps per stage");
@@ -95,11 +99,14 @@ struct OpTile {
     } else if constexpr (kEsz == 4) {
       return ((r >> 2) & 1) << 3;
     } else if constexpr (kEsz == 2) {
-      if constexpr (ATOM == 32) return (r & 3) << 2;
+      if constexpr (kRB == 128) return ((r >> 1) & 1) << 2;
+      else if constexpr (ATOM == 32) return (r & 3) << 2;
       else return ((r & 3) | (((r >> 3) & 1) << 2)) << 1;
     } else if constexpr (kRB >= 256) {
       if constexpr (ATOM == 32) return (r & 7) << 1;
       else return (r & 7) | (((r / kLaneK) & 1) << 3);
+    } else if constexpr (kRB == 64) {
+      return ((r >> 2) & 1) << 1;
     } else {
       if constexpr (ATOM == 32) return ((r >> 1) & 3) << 1;
       else return ((r >> 1) & 3) | (((r / kLaneK) & 1) << 2);

@@ -582,7 +582,7 @@ static hipError_t launch_w4_split(const GemmArgs& g, int slices, int64_t kb_slic
                      (int64_t)g.m * g.n * 4);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
-  return gemm_splitk_sum((const float*)ws, slices, g, stream);
+  return gemm_splitk_sum(ws, slices, g.n, g, stream);
 }
 
 template <bool AM, bool BM>

@@ -61,9 +61,11 @@ inline MfmaChoice gemm_mfma_choice(const GemmArgs& g, int cus, bool workspace) {
 // the plan's bytes (16-byte aligned) the planned split runs; otherwise the
 // unsplit kernels.
 hipError_t gemm_mfma(const GemmArgs& g, hipStream_t s, void* workspace, int64_t workspace_bytes);
-// C (+)= the sum over slices of partial[slice][M][N] (f32, added in slice
-// order), converted to C's type; N is a multiple of 4.
-hipError_t gemm_splitk_sum(const float* partial, int slices, const GemmArgs& g, hipStream_t s);
+// C (+)= scale times the sum over slices of partial[slice][M][pitch] (f32, or
+// i32 for an i32 C; added in slice order), converted to C's type; pitch is a
+// multiple of 4.
+hipError_t gemm_splitk_sum(const void* partial, int slices, int64_t pitch, const GemmArgs& g,
+                           hipStream_t s);
 // The kernels of one storage order (AM: A stored [K, M]; BM: B stored
 // [K, N]), instantiated in gemm_w4_a*b*.hip (256x256 tiles) and
 // gemm_128_a*b*.hip (128x128 tiles).  The split variants run `slices` K
@@ -85,8 +87,11 @@ template <bool AM, bool BM> hipError_t gemm_128_grid_layout(const GemmArgs& g, h
 template <bool AM, bool BM>
 hipError_t gemm_128_split_layout(const GemmArgs& g, int slices, int64_t kb_slice, void* ws,
                                  hipStream_t s);
-// Any layout / shape; LDS-tiled FMA kernel.
-hipError_t gemm_generic_any(const GemmArgs& g, hipStream_t s);
+// Any alignment, pitch and shape (gemm_any.h); with a workspace of at least
+// the plan's bytes the planned split runs.
+hipError_t gemm_any(const GemmArgs& g, hipStream_t s, void* workspace, int64_t workspace_bytes);
+template <bool AM, bool BM>
+hipError_t gemm_any_layout(const GemmArgs& g, const plan::SplitPlan& p, void* ws, hipStream_t s);
 // Small-M kernel (plan::skinny_supported: M <= kSkinnyMaxM, bf16/f16,
 // trans_a == 0, trans_b == 1, 16 B aligned K-contiguous rows);
 // memory-bound regime.

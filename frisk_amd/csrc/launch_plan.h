@@ -167,6 +167,49 @@ inline SplitPlan split_plan(const GemmShape& g, int cus) {
   return p;
 }
 
+// ---------------------------------------------------------------------------
+// The any-alignment kernel (gemm_any.h): 128x128 tiles (big) or 64x64, K
+// slices on stage boundaries (128 bytes), 32-bit partials of every type pair
+// in rows of any_partial_pitch elements, summed by a second launch.  The
+// choice with the least estimated time: whole rounds of tiles over the CUs at
+// the time a stage takes a CU (us, measured: 0.70 and 0.28; f32, whose MFMA
+// is 16 times slower, 1.9 and 0.48), and for a split the partials' traffic and
+// about 5 us of second launch and scratch (9x897x528: 8.0 us unsplit, 12.6
+// split).  Measured, us, over tiles and slices: 1111x3333x1777 f16 35.5 on
+// 128 tiles, 45.5 on 64; 33x189x896 16.9 and 9.1; 1589x256x13953 fp8 172 and
+// 75; 2x210x13418 153 and 64 unsplit, 13.8 and 12.4 in 32 slices.  The
+// partials stay within the scratch of frisk_gemm_noalloc.
+// ---------------------------------------------------------------------------
+inline int64_t any_partial_pitch(int64_t n) { return (n + 3) & ~(int64_t)3; }
+constexpr int64_t kAnyMaxPartial = 64ll << 20;
+
+inline SplitPlan any_plan(const GemmShape& g, int cus, bool workspace) {
+  const int64_t kb = g.k * dtype_bytes(g.in);
+  const int64_t stage = g.in == kE4M3 ? 64 : 128;  // bytes of K (e4m3 takes twice its size in LDS)
+  const int64_t slice_bytes = g.m * any_partial_pitch(g.n) * 4;
+  const int64_t chunks = (kb + 127) / 128;
+  const int64_t most = workspace ? std::min<int64_t>({chunks / 4, 64, kAnyMaxPartial / slice_bytes}) : 1;
+  SplitPlan best{1, kb, 0, false};
+  double best_us = -1.0;
+  for (const int64_t bt : {64, 128}) {
+    const int64_t tiles = ((g.m + bt - 1) / bt) * ((g.n + bt - 1) / bt);
+    const double stage_us = g.in == kF32 ? (bt == 64 ? 0.48 : 1.9) : bt == 64 ? 0.28 : 0.70;
+    // (Few candidates: the plan is made on every call.)
+    for (const int64_t sl : {1, 2, 3, 4, 6, 8, 12, 16, 24, 32, 48, 64}) {
+      if (sl > std::max<int64_t>(most, 1)) break;
+      const int64_t kb_slice = sl == 1 ? kb : (chunks + sl - 1) / sl * 128;
+      const int64_t slices = (kb + kb_slice - 1) / kb_slice;
+      if (slices < sl) continue;
+      const double us = rounds(tiles * slices, cus) * (double)((kb_slice + stage - 1) / stage) * stage_us +
+                        (slices > 1 ? 5.0 + (double)slices * slice_bytes * 2 / (kPartialBw * 1e-6) : 0.0);
+      if (best_us >= 0 && us >= best_us) continue;
+      best_us = us;
+      best = SplitPlan{(int)slices, kb_slice, slices > 1 ? slices * slice_bytes : 0, bt == 128};
+    }
+  }
+  return best;
+}
+
 // A requested variant with `slices` K slices (tile 256 or 128 with the 2x2
 // wave grid, bf16/f16/f32): the slices start on stage boundaries as the
 // library's own split would place them.
@@ -325,7 +368,7 @@ inline int64_t workspace_bytes(const GemmShape& g, Route r, int cus) {
   }
   if (r == Route::Mfma) return g.tile ? requested_split(g, cus).workspace_bytes
                                       : split_plan(g, cus).workspace_bytes;
-  return 0;
+  return any_plan(g, cus, true).workspace_bytes;
 }
 
 enum class Kernel { Generic, Skinny, W4, T128 };
@@ -354,9 +397,14 @@ inline GemmLaunch launch_of(const GemmShape& g, Route r, int cus, int64_t worksp
   L.requested = g.tile != 0;
   if (r == Route::Generic) {
     L.kernel = Kernel::Generic;
-    L.tile_m = L.tile_n = 64;
-    L.slices = 1;
-    L.kb_slice = g.k * dtype_bytes(g.in);
+    const SplitPlan p = any_plan(g, cus, ws);
+    L.tile_m = L.tile_n = p.big ? 128 : 64;
+    L.wave_m = L.wave_n = 2;
+    L.stage_bytes = 128;
+    L.slices = p.slices;
+    L.kb_slice = p.kb_slice;
+    L.slice_sum = p.slices > 1 ? SliceSum::SecondLaunch : SliceSum::None;
+    L.workspace_bytes = p.workspace_bytes;
     return L;
   }
   if (r == Route::Skinny && !(ws && g.m > kSkinnySplitMaxM)) {

@@ -132,7 +132,10 @@ int frisk_gemm(const frisk_gemm_desc* desc, void* stream);
  * bases and row pitches, K * esize is a multiple of 16 for an operand stored
  * K-contiguous (A without trans_a, B with trans_b), C's row pitch is a
  * multiple of 16 bytes, and every buffer a tile addresses spans less than
- * 2^31 bytes; anything else runs a correct but slower generic kernel. */
+ * 2^31 bytes.  Anything else ("gemm_generic" in frisk_gemm_plan) runs a
+ * matrix-core kernel that takes any alignment and pitch and stages through
+ * registers, at about half the rate; it splits K over a workspace like the
+ * others, and runs unsplit where a given workspace is short or misaligned. */
 
 /* frisk_gemm without any device allocation by the library or the caller:
  * no hipMalloc, hipFree or allocating library routine is called.  No
