@@ -636,9 +636,18 @@ static hipError_t launch_attn_kt(const AttnArgs& a, hipStream_t stream) {
   }
 }
 
-// K stored [.., seq, head_dim] or [.., head_dim, seq] (a.k_dmajor).
+// Few queries (attn_fewq.h).
+template <Elt T, Elt OUT, int D, bool CAUSAL, bool KT>
+static hipError_t launch_fewq(const AttnArgs& a, hipStream_t stream);
+
+// K stored [.., seq, head_dim] or [.., head_dim, seq] (a.k_dmajor).  Up to
+// kFewQ queries run one query tile whose waves divide the keys, whatever
+// `waves` names.
 template <Elt T, Elt OUT, int D, bool CAUSAL>
 static hipError_t launch_attn(const AttnArgs& a, hipStream_t stream) {
+  if (a.seq_q <= plan::kFewQ)
+    return a.k_dmajor ? launch_fewq<T, OUT, D, CAUSAL, true>(a, stream)
+                      : launch_fewq<T, OUT, D, CAUSAL, false>(a, stream);
   return a.k_dmajor ? launch_attn_kt<T, OUT, D, CAUSAL, true>(a, stream)
                     : launch_attn_kt<T, OUT, D, CAUSAL, false>(a, stream);
 }

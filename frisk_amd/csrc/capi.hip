@@ -405,8 +405,13 @@ int frisk_gemm(const frisk_gemm_desc* d, void* stream) {
   return launch_gemm(g, route, ws, ws_bytes, stream, "frisk_gemm");
 }
 
-int frisk_attn_fwd(const frisk_attn_desc* d, void* stream) {
-  g_last_error.clear();
+}  // extern "C"
+
+namespace {
+
+// Checks of the attention entries and the kernel arguments; 0 or an error
+// code.  With ptrs == false the tensors are not required.
+int check_attn(const frisk_attn_desc* d, bool ptrs, frisk::AttnArgs& a) {
   if (!d) return fail(FRISK_EINVAL, "frisk_attn_fwd: null descriptor");
   if (d->batch <= 0 || d->heads <= 0 || d->seq_q <= 0 || d->seq_k <= 0 || d->head_dim <= 0)
     return fail(FRISK_EINVAL, "frisk_attn_fwd: sizes must be positive");
@@ -419,7 +424,7 @@ int frisk_attn_fwd(const frisk_attn_desc* d, void* stream) {
   if (d->head_dim != 16 && d->head_dim != 32 && d->head_dim != 64 && d->head_dim != 128)
     return fail(FRISK_EUNSUP, "frisk_attn_fwd: head_dim %lld not supported (16, 32, 64, 128)",
                 (long long)d->head_dim);
-  if (!d->q || !d->k || !d->v || !d->o) return fail(FRISK_EINVAL, "frisk_attn_fwd: null tensor");
+  if (ptrs && (!d->q || !d->k || !d->v || !d->o)) return fail(FRISK_EINVAL, "frisk_attn_fwd: null tensor");
   if (!aligned16(d->q) || !aligned16(d->k) || !aligned16(d->v) || !aligned16(d->o))
     return fail(FRISK_EINVAL, "frisk_attn_fwd: Q/K/V/O must be 16-byte aligned");
   const int64_t strides[12] = {d->q_stride_b, d->q_stride_h, d->q_stride_s,
@@ -467,7 +472,6 @@ int frisk_attn_fwd(const frisk_attn_desc* d, void* stream) {
                               "2^31 - 1 bytes the kernel addresses",
                 (long long)kv_reach);
 
-  frisk::AttnArgs a;
   a.dtype = (frisk::Elt)d->dtype;
   a.out = (frisk::Elt)d->o_dtype;
   a.batch = d->batch; a.heads = d->heads; a.seq_q = d->seq_q; a.seq_k = d->seq_k;
@@ -481,10 +485,49 @@ int frisk_attn_fwd(const frisk_attn_desc* d, void* stream) {
   a.v = d->v; a.v_sb = d->v_stride_b; a.v_sh = d->v_stride_h; a.v_ss = d->v_stride_s;
   a.o = d->o; a.o_sb = d->o_stride_b; a.o_sh = d->o_stride_h; a.o_ss = d->o_stride_s;
   a.lse = d->lse;
+  return FRISK_OK;
+}
+
+int64_t attn_workspace(const frisk::AttnArgs& a) {
+  return frisk::plan::attn_workspace(a.batch * a.heads, a.seq_q, a.seq_k, a.head_dim,
+                                     frisk::device_cus());
+}
+
+}  // namespace
+
+extern "C" {
+
+int64_t frisk_attn_workspace_size(const frisk_attn_desc* d) {
+  g_last_error.clear();
+  frisk::AttnArgs a;
+  const int rc = check_attn(d, false, a);
+  return rc ? rc : attn_workspace(a);
+}
+
+int frisk_attn_fwd_ws(const frisk_attn_desc* d, void* workspace, int64_t workspace_bytes,
+                      void* stream) {
+  g_last_error.clear();
+  frisk::AttnArgs a;
+  const int rc = check_attn(d, true, a);
+  if (rc) return rc;
+  if (workspace_bytes < 0) return fail(FRISK_EINVAL, "frisk_attn_fwd: negative workspace_bytes");
+  const int64_t need = workspace ? attn_workspace(a) : 0;
+  if (need > 0) {
+    if (workspace_bytes < need)
+      return fail(FRISK_EINVAL, "frisk_attn_fwd: workspace of %lld bytes, this call takes %lld",
+                  (long long)workspace_bytes, (long long)need);
+    if (!aligned16(workspace))
+      return fail(FRISK_EINVAL, "frisk_attn_fwd: workspace must be 16-byte aligned");
+    a.workspace = workspace;
+  }
   clear_stale_error();
   hipError_t e = frisk::attn_fwd(a, (hipStream_t)stream);
   if (e != hipSuccess) return hip_fail(e, "frisk_attn_fwd launch");
   return FRISK_OK;
+}
+
+int frisk_attn_fwd(const frisk_attn_desc* d, void* stream) {
+  return frisk_attn_fwd_ws(d, nullptr, 0, stream);
 }
 
 }  // extern "C"

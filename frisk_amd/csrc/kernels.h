@@ -122,6 +122,8 @@ struct AttnArgs {
   void* o;
   int64_t o_sb, o_sh, o_ss;
   float* lse;
+  // Scratch of the key splits (plan::attn_workspace bytes) or null: unsplit.
+  void* workspace = nullptr;
 };
 
 hipError_t attn_fwd_d128(const AttnArgs& a, hipStream_t s);

@@ -487,5 +487,44 @@ inline int attn_waves(int64_t batch_heads, int64_t seq_q, int64_t head_dim, bool
   return t4 < t8 ? 4 : 8;
 }
 
+// Few queries (decode steps): up to kFewQ, one query tile, run the kernel
+// whose waves divide the keys (attn_fewq.h) in `attn_splits` key splits per
+// head, combined by a second launch from the f32 rows of attn_workspace.
+// A workgroup's round of key blocks (64 keys per wave) takes about 2.2 us of
+// a CU, all of K and V at least their bytes at 6 TB/s, a split about 5 us of
+// second launch and scratch and 0.15 us to read each split's rows.  Measured, us, 1 -> the chosen splits -> twice
+// that: b1 h32 s4096 d128 31.4 -> 16.7 (4) -> 18.4; b1 h1 s32768 d128 217 ->
+// 22.3 (32); b4 h32 s4096 d128 50.6 (1) -> 51.1; b5 h16 s2432 d64 11.9 (1) ->
+// 13.0.  (The kernel before, whose waves did not divide the keys: 81 us at b4
+// h32 s4096, 29.3 at b5 h16 s2432 d64, 48.2 at b64 h4 s5231 d16, now 16.6.)
+constexpr int64_t kFewQ = 32;
+
+inline int attn_splits(int64_t batch_heads, int64_t seq_q, int64_t seq_k, int64_t head_dim, int cus) {
+  const int64_t nkb = (seq_k + 63) / 64;
+  const int64_t waves = head_dim == 128 ? 4 : head_dim == 64 ? 8 : 16;
+  // (Up to 12 key blocks no split gains: callers ask for a workspace past
+  // that only.)
+  if (nkb <= 12) return 1;
+  const double bytes_us = 4.0 * batch_heads * seq_k * head_dim / 6e6;
+  int best = 1;
+  double best_us = -1.0;
+  for (const int s : {1, 2, 3, 4, 6, 8, 12, 16, 24, 32, 48, 64}) {
+    if (s > 1 && nkb < 2 * s) break;
+    const int64_t per = ((nkb + s - 1) / s + waves - 1) / waves;
+    const double us = std::max(rounds(batch_heads * s, cus) * (double)per * 2.2, bytes_us) +
+                      (s > 1 ? 5.0 + 0.15 * s + 8.0 * batch_heads * s * seq_q * head_dim / (kPartialBw * 1e-6) : 0.0);
+    if (best_us >= 0 && us >= best_us) continue;
+    best_us = us;
+    best = s;
+  }
+  return best;
+}
+inline int64_t attn_workspace(int64_t batch_heads, int64_t seq_q, int64_t seq_k, int64_t head_dim,
+                              int cus) {
+  if (seq_q > kFewQ) return 0;
+  const int64_t s = attn_splits(batch_heads, seq_q, seq_k, head_dim, cus);
+  return s > 1 ? batch_heads * s * seq_q * (head_dim + 2) * 4 : 0;
+}
+
 }  // namespace plan
 }  // namespace frisk

@@ -21,7 +21,7 @@ DTYPE_NAMES = {F32: "f32", F16: "f16", BF16: "bf16", E4M3: "e4m3", I8: "i8", I32
 
 # Exported symbols declared by include/frisk_hip.h.
 EXPORTS = ("frisk_gemm", "frisk_gemm_workspace_size", "frisk_gemm_plan", "frisk_gemm_noalloc",
-           "frisk_attn_fwd",
+           "frisk_attn_fwd", "frisk_attn_fwd_ws", "frisk_attn_workspace_size",
            "frisk_reduce", "frisk_reduce_workspace_size",
            "frisk_copy", "frisk_fill",
            "frisk_last_error", "frisk_abi_version", "frisk_probe_mfma_layout",
@@ -119,6 +119,11 @@ def load() -> ctypes.CDLL:
     lib.frisk_gemm_noalloc.restype = ctypes.c_int
     lib.frisk_attn_fwd.argtypes = [ctypes.POINTER(AttnDesc), ctypes.c_void_p]
     lib.frisk_attn_fwd.restype = ctypes.c_int
+    lib.frisk_attn_fwd_ws.argtypes = [ctypes.POINTER(AttnDesc), ctypes.c_void_p, ctypes.c_int64,
+                                      ctypes.c_void_p]
+    lib.frisk_attn_fwd_ws.restype = ctypes.c_int
+    lib.frisk_attn_workspace_size.argtypes = [ctypes.POINTER(AttnDesc)]
+    lib.frisk_attn_workspace_size.restype = ctypes.c_int64
     lib.frisk_reduce.argtypes = [ctypes.POINTER(ReduceDesc), ctypes.c_void_p]
     lib.frisk_reduce.restype = ctypes.c_int
     lib.frisk_reduce_workspace_size.argtypes = [ctypes.POINTER(ReduceDesc)]
@@ -339,6 +344,11 @@ def attn_desc(q, k, v, o, *, causal=False, sm_scale=None, lse=None,
                     int(bool(k_transposed)), int(waves))
 
 
+# frisk_attn_fwd_ws splits the keys of calls with at most FEW_QUERIES queries
+# and more than FEW_KEYS keys.
+FEW_QUERIES, FEW_KEYS = 32, 768
+
+
 def attn_fwd(q, k, v, o, *, causal=False, sm_scale=None, lse=None, stream=None,
              k_transposed=False, waves=0):
     """O = softmax(sm_scale . Q K^T [causal mask]) V on the GPU.  K is
@@ -347,8 +357,18 @@ def attn_fwd(q, k, v, o, *, causal=False, sm_scale=None, lse=None, stream=None,
     workgroup shape; 0 lets the library choose."""
     d = attn_desc(q, k, v, o, causal=causal, sm_scale=sm_scale, lse=lse, k_transposed=k_transposed,
                   waves=waves)
-    _check(load().frisk_attn_fwd(ctypes.byref(d), ctypes.c_void_p(_stream_handle(stream))),
-           "frisk_attn_fwd")
+    lib, ws, need = load(), None, 0
+    if d.seq_q <= FEW_QUERIES and d.seq_k > FEW_KEYS:
+        need = lib.frisk_attn_workspace_size(ctypes.byref(d))
+        _check(int(need) if need < 0 else OK, "frisk_attn_fwd")
+    if need > 0:
+        import torch
+        ws = torch.empty(need, dtype=torch.uint8, device=o.device)
+        rc = lib.frisk_attn_fwd_ws(ctypes.byref(d), ws.data_ptr(), need,
+                                   ctypes.c_void_p(_stream_handle(stream)))
+    else:
+        rc = lib.frisk_attn_fwd(ctypes.byref(d), ctypes.c_void_p(_stream_handle(stream)))
+    _check(rc, "frisk_attn_fwd")
     return o
 
 

@@ -222,6 +222,21 @@ typedef struct frisk_attn_desc {
 
 int frisk_attn_fwd(const frisk_attn_desc* desc, void* stream);
 
+/* frisk_attn_fwd with optional device scratch (16-byte aligned) owned by the
+ * caller.  A call with few queries (seq_q <= 32, a decode step) and few heads,
+ * given at least frisk_attn_workspace_size() bytes, splits the keys over the
+ * whole GPU (f32 partial rows, combined in split order by a second launch, so
+ * the same inputs give the same bits); without it, or when the size is 0, it
+ * is frisk_attn_fwd.  The contents before a call do not matter; calls that
+ * share a workspace must not overlap. */
+int frisk_attn_fwd_ws(const frisk_attn_desc* desc, void* workspace, int64_t workspace_bytes,
+                      void* stream);
+
+/* Workspace bytes that make frisk_attn_fwd_ws(desc) split the keys (0: none
+ * is used), or a negative FRISK_E* code for an invalid descriptor.  Pointers
+ * in desc are not read. */
+int64_t frisk_attn_workspace_size(const frisk_attn_desc* desc);
+
 /* Reduction kinds (frisk.reduce "add"/"max"/"min", reduce_tensor "sum"/...). */
 typedef enum frisk_reduce_kind {
   FRISK_REDUCE_SUM = 0,
