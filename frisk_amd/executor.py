@@ -600,7 +600,9 @@ def _checked_variant(p: "GemmPlan", a, b, c):
     if p.variant is None:
         return None
     try:
-        rt.gemm_plan(a, b, c, trans_a=p.trans_a, trans_b=p.trans_b, variant=p.variant)
+        # The size query makes the checks of the call, tensor alignment among them.
+        d = rt.gemm_desc(a, b, c, trans_a=p.trans_a, trans_b=p.trans_b, variant=p.variant)
+        rt.workspace_bytes_of(d)
     except ValueError as e:
         p.mismatch = f"variant {p.variant} does not run on these tensors ({e}); the library's own " \
                      "choice runs"

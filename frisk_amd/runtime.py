@@ -210,12 +210,16 @@ def gemm_desc(a, b, c, *, trans_a=False, trans_b=False, clear_accum=True,
                     int(variant[3]) if variant and len(variant) > 3 else 0)
 
 
-def gemm_workspace_bytes(a, b, c, *, trans_a=False, trans_b=False) -> int:
-    """frisk_gemm_workspace_size for gemm(a, b, c, ...): 0 when no split-K applies."""
-    d = gemm_desc(a, b, c, trans_a=trans_a, trans_b=trans_b)
-    need = int(load().frisk_gemm_workspace_size(ctypes.byref(d)))
+def workspace_bytes_of(desc: GemmDesc) -> int:
+    """frisk_gemm_workspace_size for a descriptor."""
+    need = int(load().frisk_gemm_workspace_size(ctypes.byref(desc)))
     _check(need if need < 0 else OK, "frisk_gemm_workspace_size")
     return need
+
+
+def gemm_workspace_bytes(a, b, c, *, trans_a=False, trans_b=False) -> int:
+    """frisk_gemm_workspace_size for gemm(a, b, c, ...): 0 when no split-K applies."""
+    return workspace_bytes_of(gemm_desc(a, b, c, trans_a=trans_a, trans_b=trans_b))
 
 
 def plan_of(desc: GemmDesc) -> dict:
