@@ -283,6 +283,16 @@ const char* mfma_atom(frisk::Elt in) {
   }
 }
 
+// The 16x16 MFMA of the small-M kernel.
+const char* skinny_atom(frisk::Elt in) {
+  switch (in) {
+    case frisk::Elt::BF16: return "v_mfma_f32_16x16x32_bf16";
+    case frisk::Elt::F16: return "v_mfma_f32_16x16x32_f16";
+    case frisk::Elt::E4M3: return "v_mfma_f32_16x16x32_fp8_fp8";
+    default: return "v_mfma_i32_16x16x64_i8";
+  }
+}
+
 // Launches a validated GEMM on its route with an optional split-K scratch.
 int launch_gemm(const frisk::GemmArgs& g, GemmRoute route, void* ws, int64_t ws_bytes,
                 void* stream, const char* fn) {
@@ -346,10 +356,10 @@ int frisk_gemm_plan(const frisk_gemm_desc* d, char* buf, int64_t len) {
   } else if (L.kernel == frisk::plan::Kernel::Skinny) {
     n = snprintf(buf, (size_t)len,
                  "{\"kernel\": \"gemm_skinny\", \"tile_m\": %d, \"tile_n\": %d, "
-                 "\"atom\": \"v_mfma_f32_16x16x32_%s\", \"waves\": [1, 1], \"a_major\": \"k\", "
+                 "\"atom\": \"%s\", \"waves\": [1, 1], \"a_major\": \"k\", "
                  "\"b_major\": \"k\", \"slices\": %d, \"slice_sum\": \"%s\", "
                  "\"workspace_bytes\": %lld}",
-                 L.tile_m, L.tile_n, d->a_type == FRISK_BF16 ? "bf16" : "f16", L.slices, slice_sum,
+                 L.tile_m, L.tile_n, skinny_atom(g.in), L.slices, slice_sum,
                  (long long)L.workspace_bytes);
   } else {
     const bool big = L.kernel == frisk::plan::Kernel::W4;

@@ -10,7 +10,8 @@
 //  * Operands go straight from global memory into MFMA registers (no LDS):
 //    v_mfma_f32_16x16x32_{bf16,f16} wants lane l to hold 16 contiguous bytes
 //    of row l%16 at k-offset 8*(l/16), i.e. 16 B per lane and 64 B per row
-//    per load instruction.  Batches of U k-steps are double-buffered: batch
+//    per load instruction; 8-bit types take the same 64 bytes (fp8 as two
+//    MFMAs of K 32, int8 as one of K 64).  Batches of U k-steps are double-buffered: batch
 //    b+1 is loaded while batch b is multiplied (operands from HBM:
 //    64x4096x4096 33.0 -> 24.5 us, 16x4096x4096 13.9 -> 11.9 us).
 //  * A batch of kSkinnyWaves * U k-steps gives wave w the k-step pairs
@@ -31,6 +32,12 @@
 //    slice order (deterministic) and converts.  Wider column tiles then cut
 //    the number of times X is streamed from L2 (every workgroup reads the
 //    X rows of its K range), and the slices restore the parallelism.
+//  * 8-bit types (M <= 64, never split: plan::skinny_plan).  Against 128x128
+//    tiles, which they ran on before, operands from HBM, us: fp8 32x8192x8192
+//    29.0 -> 17.2, 16x4096x4096 16.1 -> 8.1, 16x4096x14336 47.8 -> 14.5; int8
+//    16x14336x4096 16.6 -> 12.7, 64x4096x4096 16.9 -> 10.1.  What bounds them
+//    now is X, which every workgroup reads whole through L2 beside its W (the
+//    same with 8 or 16 waves per workgroup).
 //  * Roofline: HBM-bound; algorithmic bytes = M.K.2 + N.K.2 + M.N.2.
 
 #include <algorithm>
@@ -44,19 +51,39 @@ namespace {
 
 typedef float f32x4_ __attribute__((ext_vector_type(4)));
 
+// One 64-byte k-step: the 16 bytes of each lane.
 template <Elt E> struct Mfma16;
 template <> struct Mfma16<Elt::BF16> {
+  using Acc = f32x4_;
   __device__ static inline f32x4_ run(i32x4 a, i32x4 b, f32x4_ c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a),
                                                    __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
   }
 };
 template <> struct Mfma16<Elt::F16> {
+  using Acc = f32x4_;
   __device__ static inline f32x4_ run(i32x4 a, i32x4 b, f32x4_ c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a),
                                                   __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
   }
 };
+// fp8: two of K 32, the low and the high 8 bytes of A and B alike.
+template <> struct Mfma16<Elt::E4M3> {
+  using Acc = f32x4_;
+  __device__ static inline f32x4_ run(i32x4 a, i32x4 b, f32x4_ c) {
+    typedef long i64x2 __attribute__((ext_vector_type(2)));
+    const i64x2 av = __builtin_bit_cast(i64x2, a), bv = __builtin_bit_cast(i64x2, b);
+    c = __builtin_amdgcn_mfma_f32_16x16x32_fp8_fp8(av[0], bv[0], c, 0, 0, 0);
+    return __builtin_amdgcn_mfma_f32_16x16x32_fp8_fp8(av[1], bv[1], c, 0, 0, 0);
+  }
+};
+template <> struct Mfma16<Elt::I8> {
+  using Acc = i32x4;
+  __device__ static inline i32x4 run(i32x4 a, i32x4 b, i32x4 c) {
+    return __builtin_amdgcn_mfma_i32_16x16x64_i8(a, b, c, 0, 0, 0);
+  }
+};
+
 
 constexpr int kSkinnyWaves = 4;
 
@@ -75,11 +102,13 @@ template <int TM, int TN> constexpr int skinny_unroll() {
 template <Elt IN, Elt OUT, int TM, int TN>
 __global__ __launch_bounds__(64 * kSkinnyWaves) void gemm_skinny_kernel(
     const char* __restrict__ A, const char* __restrict__ B, void* __restrict__ C, int M, int N,
-    int Kb, int64_t lda_b, int64_t ldb_b, int64_t ldc, int accumulate, int steps_per_slice,
-    float* __restrict__ partial) {
+    int Kb, int64_t lda_b, int64_t ldb_b, int64_t ldc, float scale, int accumulate,
+    int steps_per_slice, void* __restrict__ partial) {
 #if defined(__HIP_DEVICE_COMPILE__)
   constexpr int U = skinny_unroll<TM, TN>();
-  __shared__ float red[kSkinnyWaves][TM * TN * 4][64];
+  using Acc = typename Mfma16<IN>::Acc;
+  using AccS = typename std::conditional<IN == Elt::I8, int32_t, float>::type;
+  __shared__ AccS red[kSkinnyWaves][TM * TN * 4][64];
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int l16 = lane & 15, quad = lane >> 4;
@@ -101,11 +130,11 @@ __global__ __launch_bounds__(64 * kSkinnyWaves) void gemm_skinny_kernel(
   // W rows past N are not clamped: the buffer range check zero-fills the
   // last tile's missing rows.
 
-  f32x4_ acc[TM][TN];
+  Acc acc[TM][TN];
 #pragma unroll
   for (int i = 0; i < TM; ++i)
 #pragma unroll
-    for (int j = 0; j < TN; ++j) acc[i][j] = f32x4_{0, 0, 0, 0};
+    for (int j = 0; j < TN; ++j) acc[i][j] = Acc{0, 0, 0, 0};
 
   // This workgroup's k-steps (64 B of K each): [s_begin, s_begin + nsteps),
   // walked from a per-workgroup offset `rot`.
@@ -168,7 +197,7 @@ __global__ __launch_bounds__(64 * kSkinnyWaves) void gemm_skinny_kernel(
   constexpr int kElems = TM * TN * 4 * 64;
   for (int e = tid; e < kElems; e += 64 * kSkinnyWaves) {
     const int idx = e >> 6, ln = e & 63;
-    float v = 0.0f;
+    AccS v = 0;
 #pragma unroll
     for (int w = 0; w < kSkinnyWaves; ++w) v += red[w][idx][ln];
     const int tile = idx >> 2, r = idx & 3;
@@ -177,11 +206,15 @@ __global__ __launch_bounds__(64 * kSkinnyWaves) void gemm_skinny_kernel(
     const int col = n0 + j * 16 + (ln & 15);
     if (row < M && col < N) {
       if (partial) {
-        partial[((int64_t)blockIdx.z * M + row) * N + col] = v;
+        ((AccS*)partial)[((int64_t)blockIdx.z * M + row) * N + col] = v;
+      } else if constexpr (OUT == Elt::I32) {
+        int32_t* c = (int32_t*)C + (int64_t)row * ldc + col;
+        *c = accumulate ? *c + v : v;
       } else {
         const int64_t o = (int64_t)row * ldc + col;
-        if (accumulate) v += load_as_f32<OUT>(C, o);
-        store_from_f32<OUT>(C, o, v);
+        float f = v * scale;
+        if (accumulate) f += load_as_f32<OUT>(C, o);
+        store_from_f32<OUT>(C, o, f);
       }
     }
   }
@@ -225,7 +258,7 @@ __global__ __launch_bounds__(256) void gemm_splitk_sum_kernel(const void* __rest
 namespace {
 
 template <Elt IN, Elt OUT, int TM, int TN>
-hipError_t launch_skinny(const GemmArgs& g, const SkinnyPlan& p, float* partial,
+hipError_t launch_skinny(const GemmArgs& g, const SkinnyPlan& p, void* partial,
                          hipStream_t stream) {
   constexpr int kEsz = EltInfo<IN>::bytes;
   dim3 grid((unsigned)((g.n + 16 * TN - 1) / (16 * TN)), (unsigned)((g.m + 16 * TM - 1) / (16 * TM)),
@@ -233,15 +266,15 @@ hipError_t launch_skinny(const GemmArgs& g, const SkinnyPlan& p, float* partial,
   const int steps = partial ? p.steps_per_slice : (int)((g.k * kEsz + 63) / 64);
   hipLaunchKernelGGL((gemm_skinny_kernel<IN, OUT, TM, TN>), grid, dim3(64 * kSkinnyWaves), 0,
                      stream, (const char*)g.a, (const char*)g.b, g.c, (int)g.m, (int)g.n,
-                     (int)(g.k * kEsz), g.lda * kEsz, g.ldb * kEsz, g.ldc, g.accumulate, steps,
-                     partial);
+                     (int)(g.k * kEsz), g.lda * kEsz, g.ldb * kEsz, g.ldc, g.scale, g.accumulate,
+                     steps, partial);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || !partial) return e;
   return gemm_splitk_sum(partial, p.slices, g.n, g, stream);
 }
 
 template <Elt IN, Elt OUT, int TN>
-hipError_t skinny_by_m(const GemmArgs& g, const SkinnyPlan& p, float* partial, hipStream_t s) {
+hipError_t skinny_by_m(const GemmArgs& g, const SkinnyPlan& p, void* partial, hipStream_t s) {
   switch (p.tm) {
     case 1: return launch_skinny<IN, OUT, 1, TN>(g, p, partial, s);
     case 2: return launch_skinny<IN, OUT, 2, TN>(g, p, partial, s);
@@ -251,7 +284,7 @@ hipError_t skinny_by_m(const GemmArgs& g, const SkinnyPlan& p, float* partial, h
 }
 
 template <Elt IN, Elt OUT>
-hipError_t skinny_by_n(const GemmArgs& g, const SkinnyPlan& p, float* partial, hipStream_t s) {
+hipError_t skinny_by_n(const GemmArgs& g, const SkinnyPlan& p, void* partial, hipStream_t s) {
   switch (p.tn) {
     case 1: return skinny_by_m<IN, OUT, 1>(g, p, partial, s);
     case 2: return skinny_by_m<IN, OUT, 2>(g, p, partial, s);
@@ -284,10 +317,10 @@ hipError_t gemm_splitk_sum(const void* partial, int slices, int64_t pitch, const
 
 hipError_t gemm_skinny(const GemmArgs& g, hipStream_t s, void* workspace, int64_t workspace_bytes) {
   SkinnyPlan p = gemm_skinny_plan(g, device_cus(), true);
-  float* partial = nullptr;
+  void* partial = nullptr;
   if (p.slices > 1) {
     if (workspace && workspace_bytes >= p.workspace_bytes)
-      partial = (float*)workspace;
+      partial = workspace;
     else
       p = gemm_skinny_plan(g, 0, false);
   }
@@ -296,6 +329,10 @@ hipError_t gemm_skinny(const GemmArgs& g, hipStream_t s, void* workspace, int64_
     case ((int)Elt::BF16 << 8) | (int)Elt::F32: return skinny_by_n<Elt::BF16, Elt::F32>(g, p, partial, s);
     case ((int)Elt::F16 << 8) | (int)Elt::F16: return skinny_by_n<Elt::F16, Elt::F16>(g, p, partial, s);
     case ((int)Elt::F16 << 8) | (int)Elt::F32: return skinny_by_n<Elt::F16, Elt::F32>(g, p, partial, s);
+    case ((int)Elt::E4M3 << 8) | (int)Elt::BF16: return skinny_by_n<Elt::E4M3, Elt::BF16>(g, p, partial, s);
+    case ((int)Elt::E4M3 << 8) | (int)Elt::F16: return skinny_by_n<Elt::E4M3, Elt::F16>(g, p, partial, s);
+    case ((int)Elt::E4M3 << 8) | (int)Elt::F32: return skinny_by_n<Elt::E4M3, Elt::F32>(g, p, partial, s);
+    case ((int)Elt::I8 << 8) | (int)Elt::I32: return skinny_by_n<Elt::I8, Elt::I32>(g, p, partial, s);
     default: return hipErrorInvalidValue;
   }
 }

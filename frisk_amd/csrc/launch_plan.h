@@ -44,6 +44,9 @@ constexpr int64_t kSkinnyMaxM = FRISK_SKINNY_MAX_M;
 // more (up to its limit) run split on 128x128 tiles, which share each X
 // tile across the workgroup's waves through LDS.
 constexpr int64_t kSkinnySplitMaxM = 64;
+// 8-bit inputs: past 64 rows the 128x128 tiles are as fast or faster (fp8
+// 128x8192x8192 30.3 us against 39.0).
+constexpr int64_t kSkinnyMaxM8 = 64;
 // Split-K arrival words per tile of the in-launch slice sum (gemm_common.h
 // splitk_tree) and the most slices summed that way on 128x128 tiles.
 constexpr int kTreeWords = 64;
@@ -275,6 +278,7 @@ inline int stage_bytes_128(const GemmShape& g, int cus) {
 // partial tiles need (0 without split-K).
 // ---------------------------------------------------------------------------
 inline bool skinny_supported(const GemmShape& g) {
+  if (g.in == kE4M3 || g.in == kI8) return g.m <= kSkinnyMaxM8 && !g.trans_a && g.trans_b;
   const bool type_ok = (g.in == kBF16 && (g.out == kBF16 || g.out == kF32)) ||
                        (g.in == kF16 && (g.out == kF16 || g.out == kF32));
   return type_ok && g.m <= kSkinnyMaxM && !g.trans_a && g.trans_b;
@@ -289,11 +293,24 @@ inline SkinnyPlan skinny_plan(const GemmShape& g, int cus, bool split) {
   SkinnyPlan p;
   p.tm = g.m <= 16 ? 1 : g.m <= 32 ? 2 : g.m <= 64 ? 4 : 8;
   p.tn = g.n >= 8192 ? 2 : 1;  // 32-column tiles once N alone gives >= 256 of them
-  const int64_t kb = g.k * 2;   // bf16 / f16
+  const int64_t kb = g.k * dtype_bytes(g.in);
   const int64_t steps = (kb + 63) / 64;
   p.steps_per_slice = (int)steps;
   p.slices = 1;
   p.workspace_bytes = 0;
+  if (g.in == kE4M3 || g.in == kI8) {
+    // The narrowest columns whose tiles fit the CUs in one round, else the
+    // widest, unsplit (us, 16-, 32-, 64-column tiles, and two slices of the
+    // best: fp8 32x8192x8192 24.1, 17.2, 21.3, 18.4; 16x4096x4096 8.0, 8.1,
+    // 12.1, 12.3; 64x8192x8192 31, 26.1, 26.4, 26.4; int8 16x14336x4096 17.5,
+    // 13.7, 12.7, 16.8).
+    const int64_t rows = (g.m + 16 * p.tm - 1) / (16 * p.tm);
+    p.tn = 1;
+    while (p.tn < 4 && (g.n + 16 * p.tn - 1) / (16 * p.tn) * rows > (cus > 0 ? cus : 256)) p.tn *= 2;
+    // 32x32 tiles instead of 64x16: fewer loads (64x4096x4096 11.9 -> 10.1).
+    if (p.tm == 4 && p.tn == 1) p.tm = p.tn = 2;
+    return p;
+  }
   // Below 64 MiB of W the unsplit kernel ends before a second launch pays
   // (16 x 4096 x 4096: 10.5 us unsplit, 12.7 us split).
   // (The slice sum reads rows of 4 floats, so N % 4 != 0 runs unsplit too.)
