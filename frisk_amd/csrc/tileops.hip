@@ -51,53 +51,71 @@ template <> __device__ __forceinline__ float identity<kReduceMax>() { return -__
 template <> __device__ __forceinline__ float identity<kReduceMin>() { return __builtin_inff(); }
 
 // Symmetric in its operands (bitwise, NaN payloads aside), so a lane
-// exchange can evaluate one tree node on both partners.
+// exchange can evaluate one tree node on both partners.  max / min are one
+// v_maximum3_f32 / v_minimum3_f32 for up to two combines (written out in
+// compares and selects they made an 8192x16384 max along axis 0 a third
+// slower than its sum: 125 us against 97), and associative, so their order is
+// free.
 template <Elt E, int KIND>
 __device__ __forceinline__ float combine(float a, float b) {
-  if constexpr (KIND == kReduceSum) {
-    return round_to<E>(a + b);
-  } else {
-    if (a != a || b != b) return a + b;  // quiet NaN
-    const uint32_t ua = __builtin_bit_cast(uint32_t, a), ub = __builtin_bit_cast(uint32_t, b);
-    if (a == b)  // equal values; for +-0 the sign decides
-      return __builtin_bit_cast(float, KIND == kReduceMax ? (ua & ub) : (ua | ub));
-    if constexpr (KIND == kReduceMax) return a > b ? a : b;
-    else return a < b ? a : b;
-  }
+  if constexpr (KIND == kReduceSum) return round_to<E>(a + b);
+  else if constexpr (KIND == kReduceMax) return __builtin_elementwise_maximum(a, b);
+  else return __builtin_elementwise_minimum(a, b);
 }
 
-// Binary counter over a sequence of complete, equally sized subtrees: after
-// push(k, x) for k = 0..n-1, level l holds the block of 2^l subtrees for
-// every set bit l of n, and finish(n) combines them from the smallest
-// (rightmost) block up, which is the canonical tree over the sequence.
-template <Elt E, int KIND, int L>
+// Binary counter over a sequence of complete, equally sized subtrees of NV
+// outputs: after push(k, x) for k = 0..n-1, level l holds the block of 2^l
+// subtrees for every set bit l of n, and finish(n) combines them from the
+// smallest (rightmost) block up, which is the canonical tree over the
+// sequence.  k is the same in every lane, so a push takes a branch per merge,
+// two on average.  max / min keep one running value.
+template <Elt E, int KIND, int L, int NV>
 struct Counter {
-  float lvl[L];
-  // Straight-line over the levels (predicated, static indices) so that the
-  // levels stay in registers.
-  __device__ __forceinline__ void push(uint32_t k, float x) {
-    bool carry = true;
+  static constexpr bool kTree = KIND == kReduceSum;
+  float lvl[kTree ? L : 1][NV];
+  __device__ __forceinline__ void push(uint32_t k, float (&x)[NV]) {
+    if constexpr (kTree) {
+      merge<0>(__builtin_amdgcn_readfirstlane(k), x);
+    } else {
 #pragma unroll
-    for (int l = 0; l < L; ++l) {
-      const bool merge = carry && ((k >> l) & 1u);
-      if (carry && !merge) lvl[l] = x;
-      if (merge) x = combine<E, KIND>(lvl[l], x);
-      carry = merge;
+      for (int j = 0; j < NV; ++j) lvl[0][j] = k ? combine<E, KIND>(lvl[0][j], x[j]) : x[j];
     }
   }
-  __device__ __forceinline__ float finish(uint32_t n) const {
+  template <int l>
+  __device__ __forceinline__ void merge(uint32_t k, float (&x)[NV]) {
+    if constexpr (l < L) {
+      if ((k >> l) & 1u) {
+#pragma unroll
+        for (int j = 0; j < NV; ++j) x[j] = combine<E, KIND>(lvl[l][j], x[j]);
+        merge<l + 1>(k, x);
+      } else {
+#pragma unroll
+        for (int j = 0; j < NV; ++j) lvl[l][j] = x[j];
+      }
+    }
+  }
+  __device__ __forceinline__ float finish(uint32_t n, int j) const {
+    if constexpr (!kTree) return n ? lvl[0][j] : identity<KIND>();
     float t = identity<KIND>();
     bool have = false;
 #pragma unroll
-    for (int l = 0; l < L; ++l) {
+    for (int l = 0; l < (kTree ? L : 1); ++l) {
       if ((n >> l) & 1u) {
-        t = have ? combine<E, KIND>(lvl[l], t) : lvl[l];
+        t = have ? combine<E, KIND>(lvl[l][j], t) : lvl[l][j];
         have = true;
       }
     }
     return t;
   }
 };
+
+// Vectors at any (element) alignment: a global load or store takes any
+// address (32768x4095 bf16 rows, loaded by element before: 222 -> 78 us).
+// Reductions load them past the caches, each byte being read once: f32
+// 32768x4096 along axis 1 91 -> 82 us, 8192x16384 along axis 0 103 -> 93.
+typedef f32x4 f32x4_any __attribute__((aligned(1)));
+typedef i32x4 i32x4_any __attribute__((aligned(1)));
+typedef i32x2 i32x2_any __attribute__((aligned(1)));
 
 template <Elt E> __device__ __forceinline__ float load_elt(const void* p, int64_t i) {
   return load_as_f32<E>(p, i);
@@ -106,17 +124,17 @@ template <Elt E> __device__ __forceinline__ float load_elt(const void* p, int64_
 // The pairwise tree over V consecutive elements starting at column c (the
 // lowest log2(V) levels); columns at or past `cols` are the identity.
 template <Elt E, int KIND, int V>
-__device__ __forceinline__ float slot_tree(const void* row, int64_t c, int64_t cols, bool vec_ok) {
+__device__ __forceinline__ float slot_tree(const void* row, int64_t c, int64_t cols) {
   float x[V];
-  if (vec_ok && c + V <= cols) {
+  if (c + V <= cols) {
     if constexpr (E == Elt::F32) {
       static_assert(V == 4, "f32 slot");
-      const f32x4 v = *(const f32x4*)((const float*)row + c);
+            const f32x4 v = __builtin_nontemporal_load((const f32x4_any*)((const float*)row + c));
 #pragma unroll
       for (int i = 0; i < 4; ++i) x[i] = v[i];
     } else {
       static_assert(V == 8, "16-bit slot");
-      const i32x4 v = *(const i32x4*)((const uint16_t*)row + c);
+            const i32x4 v = __builtin_nontemporal_load((const i32x4_any*)((const uint16_t*)row + c));
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const uint32_t w = (uint32_t)v[i];
@@ -148,33 +166,38 @@ __device__ __forceinline__ float slot_tree(const void* row, int64_t c, int64_t c
 // index bits, then the LPR lanes of the row's lane group, then the R
 // registers.  Loads are coalesced across lanes for each r.  Chunk roots
 // (complete subtrees of S columns, the last one padded) go through a binary
-// counter.  A wave holds 64 / LPR rows.
-template <Elt E, int KIND, int R>
-__global__ __launch_bounds__(tile::kThreads) void reduce_rows_kernel(
+// counter.  A wave holds 64 / LPR rows; or, of few long rows, WPR waves share
+// one (each an aligned run of chunks_per_wave chunks, a power of two; the
+// runs' roots combine pairwise through LDS): with a wave per row 128x28653 f32
+// ran on 128 waves (109 -> 6.7 us; 384x14080 58.8 -> 6.8).
+template <Elt E, int KIND, int R, int WPR>
+__global__ __launch_bounds__(WPR > 4 ? 64 * WPR : tile::kThreads) void reduce_rows_kernel(
     const void* __restrict__ src, int64_t ld, int64_t rows, int64_t cols, void* __restrict__ dst,
-    int64_t dst_stride, int clear, int lpr_log2, int vec_ok, uint32_t chunks) {
+    int64_t dst_stride, int clear, int lpr_log2, uint32_t chunks, uint32_t chunks_per_wave) {
   using namespace tile;
   constexpr int V = 16 / EltInfo<E>::bytes;
-  const int lane = threadIdx.x & 63;
+  __shared__ float part[WPR > 1 ? WPR : 1];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int lpr = 1 << lpr_log2;
   const int lr = lane & (lpr - 1);
-  const int64_t row =
-      ((int64_t)blockIdx.x * (kThreads / 64) + (threadIdx.x >> 6)) * (64 >> lpr_log2) +
-      (lane >> lpr_log2);
+  const int64_t row = WPR > 1 ? (int64_t)blockIdx.x
+                              : ((int64_t)blockIdx.x * (kThreads / 64) + wave) * (64 >> lpr_log2) +
+                                    (lane >> lpr_log2);
   const bool live = row < rows;
   const char* rp = (const char*)src + (live ? row : 0) * ld * EltInfo<E>::bytes;
   const int64_t span = live ? cols : 0;  // dead rows load nothing
   const int64_t S = (int64_t)lpr * R * V;
+  const uint32_t k0 = WPR > 1 ? min(chunks, wave * chunks_per_wave) : 0;
+  const uint32_t n = WPR > 1 ? min(chunks, k0 + chunks_per_wave) - k0 : chunks;
 
-  Counter<E, KIND, 24> ctr;
+  Counter<E, KIND, 24, 1> ctr;
   // Every lane runs the same trip count: the lane exchanges need the whole
   // wave.
-  for (uint32_t k = 0; k < chunks; ++k) {
+  for (uint32_t k = 0; k < n; ++k) {
     float v[R];
 #pragma unroll
     for (int r = 0; r < R; ++r)
-      v[r] = slot_tree<E, KIND, V>(rp, (int64_t)k * S + ((int64_t)r * lpr + lr) * V, span,
-                                   vec_ok != 0);
+      v[r] = slot_tree<E, KIND, V>(rp, (int64_t)(k0 + k) * S + ((int64_t)r * lpr + lr) * V, span);
     for (int j = 0; j < lpr_log2; ++j) {
 #pragma unroll
       for (int r = 0; r < R; ++r) v[r] = combine<E, KIND>(v[r], __shfl_xor(v[r], 1 << j, 64));
@@ -183,89 +206,100 @@ __global__ __launch_bounds__(tile::kThreads) void reduce_rows_kernel(
     for (int w = 1; w < R; w <<= 1)
 #pragma unroll
       for (int r = 0; r < R; r += 2 * w) v[r] = combine<E, KIND>(v[r], v[r + w]);
-    ctr.push(k, v[0]);
+    float x[1] = {v[0]};
+    ctr.push(k, x);
   }
-  float res = ctr.finish(chunks);
-  if (live && lr == 0) {
+  float res = ctr.finish(n, 0);
+  if constexpr (WPR > 1) {
+    if (lane == 0) part[wave] = res;
+    __syncthreads();
+    float t[WPR];
+#pragma unroll
+    for (int w = 0; w < WPR; ++w) t[w] = part[w];
+#pragma unroll
+    for (int s = 1; s < WPR; s <<= 1)
+#pragma unroll
+      for (int w = 0; w < WPR; w += 2 * s) t[w] = combine<E, KIND>(t[w], t[w + s]);
+    res = t[0];
+  }
+  if (live && (WPR > 1 ? threadIdx.x == 0 : lr == 0)) {
     if (!clear) res = combine<E, KIND>(load_as_f32<E>(dst, row * dst_stride), res);
     store_from_f32<E>(dst, row * dst_stride, res);
   }
 }
 
 // ---- axis 0: reduce across rows -------------------------------------------------
-// A workgroup of 1024 threads owns CVB slots of 4 adjacent columns; its
-// 1024 / CVB row groups each take an aligned block of B = 2^b_log2 rows
-// (B >= 8).  The grid has one workgroup per column strip only, so the large
-// workgroup is what keeps enough loads in flight (16 waves per CU).  A thread walks
-// its block eight rows at a time: the eight-row subtree is built in
-// registers and pushed into a binary counter.  The block roots (complete
-// subtrees; an empty block is the identity) are combined in LDS by the
-// pairwise tree over the row groups.
-constexpr int kColThreads = 1024;
-
-template <Elt E, int KIND>
-__global__ __launch_bounds__(kColThreads) void reduce_cols_kernel(
+// A workgroup of T threads owns 2^cvb_log2 slots of 4 adjacent columns and the
+// rows [block B, (block + 1) B) of its blockIdx.y; its T >> cvb_log2 row groups
+// each take an aligned run of 2^b_log2 (>= 8) of them.  A thread walks its run
+// eight rows at a time: the eight-row subtree is built in registers and pushed
+// into a binary counter of LV levels.  The groups' roots (complete subtrees;
+// an empty run is the identity) are combined in LDS by the pairwise tree over
+// the groups, and go to dst, or, in the first of two passes, to
+// partial[block][column] as f32; the second pass is the same kernel over the
+// partials (LOAD f32) with the combines of E.
+template <Elt E, Elt LOAD, int KIND, int T, int LV>
+__global__ __launch_bounds__(T, T > 256 || LV <= 6 ? 4 : 1) void reduce_cols_kernel(
     const void* __restrict__ src, int64_t ld, int64_t rows, int64_t cols, void* __restrict__ dst,
-    int64_t dst_stride, int clear, int cvb_log2, int b_log2, int vec_ok) {
+    int64_t dst_stride, int clear, int cvb_log2, int b_log2, float* __restrict__ partial) {
   using namespace tile;
-  constexpr int kEsz = EltInfo<E>::bytes;
-  __shared__ float part[kColThreads * 4];
+  constexpr int kEsz = EltInfo<LOAD>::bytes;
+  __shared__ float part[T * 4];
   const int tid = threadIdx.x;
   const int cvb = 1 << cvb_log2;
   const int cs = tid & (cvb - 1), g = tid >> cvb_log2;
-  const int groups = kColThreads >> cvb_log2;
+  const int groups = T >> cvb_log2;
   const int64_t c0 = ((int64_t)blockIdx.x * cvb + cs) * 4;
-  const int64_t r0 = (int64_t)g << b_log2;
+  const int64_t r0 = ((int64_t)blockIdx.y * groups + g) << b_log2;
   const int64_t r1 = min(rows, r0 + ((int64_t)1 << b_log2));
-  const bool full = vec_ok && c0 + 4 <= cols;
+  const bool full = c0 + 4 <= cols;
 
-  Counter<E, KIND, 18> ctr[4];
+  Counter<E, KIND, LV, 4> ctr;
   uint32_t n8 = 0;
   for (int64_t i0 = r0; i0 < r1; i0 += 8, ++n8) {
     float x[8][4];
+    const char* rp = (const char*)src + (i0 * ld + c0) * kEsz;
+    if (full && i0 + 8 <= r1) {
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int64_t r = i0 + i;
-      const char* rp = (const char*)src + r * ld * kEsz;
-      if (r < r1 && full) {
-        if constexpr (E == Elt::F32) {
-          const f32x4 v = *(const f32x4*)((const float*)rp + c0);
+      for (int i = 0; i < 8; ++i) {
+        const char* p = rp + i * ld * kEsz;
+        if constexpr (LOAD == Elt::F32) {
+          const f32x4 v = __builtin_nontemporal_load((const f32x4_any*)p);
 #pragma unroll
           for (int j = 0; j < 4; ++j) x[i][j] = v[j];
         } else {
-          const uint2 v = *(const uint2*)((const uint16_t*)rp + c0);
-          const uint32_t w[2] = {v.x, v.y};
+          const i32x2 v = __builtin_nontemporal_load((const i32x2_any*)p);
 #pragma unroll
           for (int j = 0; j < 4; ++j) {
-            const uint16_t h = (uint16_t)(w[j >> 1] >> (16 * (j & 1)));
-            x[i][j] = E == Elt::BF16 ? bf16_bits_to_f32(h)
-                                     : (float)__builtin_bit_cast(_Float16, h);
+            const uint16_t h = (uint16_t)((uint32_t)v[j >> 1] >> (16 * (j & 1)));
+            x[i][j] = LOAD == Elt::BF16 ? bf16_bits_to_f32(h) : (float)__builtin_bit_cast(_Float16, h);
           }
         }
-      } else {
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
 #pragma unroll
         for (int j = 0; j < 4; ++j)
-          x[i][j] = r < r1 && c0 + j < cols ? load_as_f32<E>(rp, c0 + j) : identity<KIND>();
-      }
+          x[i][j] = i0 + i < r1 && c0 + j < cols ? load_as_f32<LOAD>(rp + i * ld * kEsz, j)
+                                                 : identity<KIND>();
     }
+    float t[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
 #pragma unroll
       for (int w = 1; w < 8; w <<= 1)
 #pragma unroll
         for (int i = 0; i < 8; i += 2 * w) x[i][j] = combine<E, KIND>(x[i][j], x[i + w][j]);
-      ctr[j].push(n8, x[0][j]);
+      t[j] = x[0][j];
     }
+    ctr.push(n8, t);
   }
 #pragma unroll
-  for (int j = 0; j < 4; ++j)
-    part[(g * cvb + cs) * 4 + j] = n8 ? ctr[j].finish(n8) : identity<KIND>();
+  for (int j = 0; j < 4; ++j) part[(g * cvb + cs) * 4 + j] = ctr.finish(n8, j);
   __syncthreads();
   // The pairwise tree over the row groups, one level at a time across the
   // workgroup: at level w group g (a multiple of 2w) takes in group g + w.
-  // The same combines as a serial walk, so the same bits; serially, one
-  // group's threads spent about 60 us on 128 groups' chains of dependent
-  // LDS accesses (33 x 777 f16).
   for (int w = 1; w < groups; w <<= 1) {
     if ((g & (2 * w - 1)) == 0) {
 #pragma unroll
@@ -281,128 +315,15 @@ __global__ __launch_bounds__(kColThreads) void reduce_cols_kernel(
       const int64_t c = c0 + j;
       if (c < cols) {
         float res = part[cs * 4 + j];
-        if (!clear) res = combine<E, KIND>(load_as_f32<E>(dst, c * dst_stride), res);
-        store_from_f32<E>(dst, c * dst_stride, res);
-      }
-    }
-  }
-}
-
-// ---- axis 0 in two passes ----------------------------------------------------------
-// Pass 1: workgroup (strip, block) reduces rows [block B, (block + 1) B) of a
-// strip of 4 * SPS columns (SPS = 2^sps_log2 <= 256 four-column slots, one
-// per lane along the columns, so a row segment of up to 4 KiB is read
-// contiguously by the whole workgroup); the 256 / SPS row groups each take
-// B / groups consecutive rows.  Group roots are combined by the pairwise
-// tree over the groups in LDS, and the block root (a complete subtree of B
-// rows; the last block padded) goes to the workspace as
-// partial[block][column].  Pass 2 combines the partials of each column in
-// block order through a binary counter.
-template <Elt E, int KIND>
-__global__ __launch_bounds__(tile::kThreads) void reduce_cols_blocks_kernel(
-    const void* __restrict__ src, int64_t ld, int64_t rows, int64_t cols, int sps_log2,
-    int b_log2, float* __restrict__ partial, int vec_ok) {
-  using namespace tile;
-  constexpr int kEsz = EltInfo<E>::bytes;
-  __shared__ float part[kThreads * 4];
-  const int tid = threadIdx.x;
-  const int sps = 1 << sps_log2;
-  const int cs = tid & (sps - 1), g = tid >> sps_log2;
-  const int groups = kThreads >> sps_log2;
-  const int64_t c0 = ((int64_t)blockIdx.x * sps + cs) * 4;
-  const int64_t gb = ((int64_t)1 << b_log2) / groups;  // rows per group, >= 8
-  const int64_t r0 = ((int64_t)blockIdx.y << b_log2) + g * gb;
-  const int64_t r1 = min(rows, r0 + gb);
-  // Four-element vector loads need the source and its rows aligned to them
-  // (element-aligned views such as x[:, 1:] take element loads).
-  const bool full = vec_ok && c0 + 4 <= cols;
-
-  // gb <= 2^12 (cols_split), so a group pushes at most 2^9 eight-row subtrees.
-  Counter<E, KIND, 10> ctr[4];
-  uint32_t n8 = 0;
-  for (int64_t i0 = r0; i0 < r1; i0 += 8, ++n8) {
-    float x[8][4];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int64_t r = i0 + i;
-      const char* rp = (const char*)src + r * ld * kEsz;
-      if (r < r1 && full) {
-        if constexpr (E == Elt::F32) {
-          const f32x4 v = *(const f32x4*)((const float*)rp + c0);
-#pragma unroll
-          for (int j = 0; j < 4; ++j) x[i][j] = v[j];
+        if (partial) {
+          partial[(int64_t)blockIdx.y * cols + c] = res;
         } else {
-          const uint2 v = *(const uint2*)((const uint16_t*)rp + c0);
-          const uint32_t w[2] = {v.x, v.y};
-#pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            const uint16_t h = (uint16_t)(w[j >> 1] >> (16 * (j & 1)));
-            x[i][j] = E == Elt::BF16 ? bf16_bits_to_f32(h) : (float)__builtin_bit_cast(_Float16, h);
-          }
+          if (!clear) res = combine<E, KIND>(load_as_f32<E>(dst, c * dst_stride), res);
+          store_from_f32<E>(dst, c * dst_stride, res);
         }
-      } else {
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-          x[i][j] = r < r1 && c0 + j < cols ? load_as_f32<E>(rp, c0 + j) : identity<KIND>();
       }
     }
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-#pragma unroll
-      for (int w = 1; w < 8; w <<= 1)
-#pragma unroll
-        for (int i = 0; i < 8; i += 2 * w) x[i][j] = combine<E, KIND>(x[i][j], x[i + w][j]);
-      ctr[j].push(n8, x[0][j]);
-    }
   }
-  if (groups == 1) {  // no exchange needed
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-      if (c0 + j < cols)
-        partial[(int64_t)blockIdx.y * cols + c0 + j] = n8 ? ctr[j].finish(n8) : identity<KIND>();
-    return;
-  }
-#pragma unroll
-  for (int j = 0; j < 4; ++j) part[(g * sps + cs) * 4 + j] = n8 ? ctr[j].finish(n8) : identity<KIND>();
-  __syncthreads();
-  // The pairwise tree over the row groups, a level at a time (as in
-  // reduce_cols_kernel).
-  for (int w = 1; w < groups; w <<= 1) {
-    if ((g & (2 * w - 1)) == 0) {
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-        part[(g * sps + cs) * 4 + j] =
-            combine<E, KIND>(part[(g * sps + cs) * 4 + j], part[((g + w) * sps + cs) * 4 + j]);
-    }
-    __syncthreads();
-  }
-  if (g == 0) {
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-      if (c0 + j < cols) partial[(int64_t)blockIdx.y * cols + c0 + j] = part[cs * 4 + j];
-  }
-}
-
-template <Elt E, int KIND>
-__global__ __launch_bounds__(tile::kThreads) void reduce_cols_final_kernel(
-    const float* __restrict__ partial, int64_t cols, uint32_t blocks, void* __restrict__ dst,
-    int64_t dst_stride, int clear) {
-  using namespace tile;
-  const int64_t c = (int64_t)blockIdx.x * kThreads + threadIdx.x;
-  if (c >= cols) return;
-  Counter<E, KIND, 24> ctr;
-  uint32_t b = 0;
-  for (; b + 8 <= blocks; b += 8) {  // eight loads in flight, then their pushes
-    float v[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) v[i] = partial[(int64_t)(b + i) * cols + c];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) ctr.push(b + i, v[i]);
-  }
-  for (; b < blocks; ++b) ctr.push(b, partial[(int64_t)b * cols + c]);
-  float res = ctr.finish(blocks);
-  if (!clear) res = combine<E, KIND>(load_as_f32<E>(dst, c * dst_stride), res);
-  store_from_f32<E>(dst, c * dst_stride, res);
 }
 
 // ---- any axis, permuted leaf order ------------------------------------------------
@@ -423,15 +344,16 @@ __global__ __launch_bounds__(tile::kThreads) void reduce_perm_kernel(
   using namespace tile;
   const int64_t o = (int64_t)blockIdx.x * kThreads + threadIdx.x;
   if (o >= outputs) return;
-  Counter<E, KIND, 32> ctr;
+  Counter<E, KIND, 32, 1> ctr;
   const uint32_t n = 1u << nb;
   for (uint32_t p = 0; p < n; ++p) {
     int64_t idx = 0;
     for (int j = 0; j < nb; ++j) idx |= (int64_t)((p >> j) & 1u) << order.bit[j];
     const int64_t off = axis == 1 ? o * ld + idx : idx * ld + o;
-    ctr.push(p, load_as_f32<E>(src, off));
+    float x[1] = {load_as_f32<E>(src, off)};
+    ctr.push(p, x);
   }
-  float res = ctr.finish(n);
+  float res = ctr.finish(n, 0);
   if (!clear) res = combine<E, KIND>(load_as_f32<E>(dst, o * dst_stride), res);
   store_from_f32<E>(dst, o * dst_stride, res);
 }
@@ -475,7 +397,7 @@ template <> __device__ __forceinline__ void put<Elt::E4M3>(void* p, int64_t i, f
 
 // Eight elements as raw bits, for vector loads and stores of 8 * esize bytes.
 template <int BYTES> struct Raw8;
-template <> struct Raw8<1> { using T = uint2; };
+template <> struct Raw8<1> { using T = i32x2; };
 template <> struct Raw8<2> { using T = i32x4; };
 template <> struct Raw8<4> { using T = i32x8; };
 template <> struct Raw8<8> { using T = i32x16; };
@@ -493,107 +415,146 @@ constexpr int kSlots = 4;  // 8-element slots per thread
 
 }  // namespace tile
 
-// Slot s of row r holds columns [8 s, 8 s + 8).  Thread t of block x works
-// on slots (x kSlots + u) 256 + t, u < kSlots, of rows y, y + gridDim.y, ...
-template <Elt S, Elt D>
+// Slot s of row r holds columns [8 s, 8 s + 8).  A thread works on kSlots of
+// them, its loads first and its stores after, so that kSlots loads are in
+// flight.  WIDE: thread t of block x takes slots (x kSlots + u) 256 + t, u <
+// kSlots, of rows y, y + gridDim.y, ...  Rows of at most 128 slots share a
+// workgroup instead, 2^tpr_log2 threads each: with a workgroup per row a
+// [30000, 136] copy kept 17 of 256 threads busy (23.3 -> 6.7 us).
+// load(u, r, c) and store(u, r, c) are called for every slot inside.
+template <bool WIDE, typename Load, typename Store>
+__device__ __forceinline__ void each_slot(int64_t rows, int64_t cols, int tpr_log2, Load load,
+                                          Store store) {
+  using namespace tile;
+  if constexpr (WIDE) {
+    for (int64_t r = blockIdx.y; r < rows; r += gridDim.y) {
+#pragma unroll
+      for (int u = 0; u < kSlots; ++u) {
+        const int64_t c = ((int64_t)(blockIdx.x * kSlots + u) * kThreads + threadIdx.x) * 8;
+        if (c < cols) load(u, r, c);
+      }
+#pragma unroll
+      for (int u = 0; u < kSlots; ++u) {
+        const int64_t c = ((int64_t)(blockIdx.x * kSlots + u) * kThreads + threadIdx.x) * 8;
+        if (c < cols) store(u, r, c);
+      }
+    }
+  } else {
+    const int rpp = kThreads >> tpr_log2;  // rows per pass of the workgroup
+    const int64_t c = (int64_t)(threadIdx.x & ((1 << tpr_log2) - 1)) * 8;
+    if (c >= cols) return;
+    const int sub = threadIdx.x >> tpr_log2;
+    for (int64_t r0 = (int64_t)blockIdx.x * rpp * kSlots; r0 < rows;
+         r0 += (int64_t)gridDim.x * rpp * kSlots) {
+#pragma unroll
+      for (int u = 0; u < kSlots; ++u)
+        if (r0 + u * rpp + sub < rows) load(u, r0 + u * rpp + sub, c);
+#pragma unroll
+      for (int u = 0; u < kSlots; ++u)
+        if (r0 + u * rpp + sub < rows) store(u, r0 + u * rpp + sub, c);
+    }
+  }
+}
+
+// Eight elements at any element alignment.
+namespace tile {
+template <typename Raw> __device__ __forceinline__ Raw load_any(const void* p) {
+  typedef Raw Any __attribute__((aligned(1)));
+  return *(const Any*)p;
+}
+template <typename Raw> __device__ __forceinline__ void store_any(void* p, const Raw& v) {
+  typedef Raw Any __attribute__((aligned(1)));
+  *(Any*)p = v;
+}
+// A copy's output: past the caches when a lane's eight elements are at most 16
+// bytes, whole lines per wave (16384x8192 bf16 -> f16 96.1 -> 92.9 us,
+// 8192x2048 f32 -> bf16 18.2 -> 15.1; as two halves of 32 bytes f32 188 ->
+// 326).
+template <typename Raw> __device__ __forceinline__ void store_stream(void* p, const Raw& v) {
+  typedef Raw Any __attribute__((aligned(1)));
+  if constexpr (sizeof(Raw) <= 16) __builtin_nontemporal_store(v, (Any*)p);
+  else *(Any*)p = v;
+}
+}  // namespace tile
+
+template <Elt S, Elt D, bool WIDE>
 __global__ __launch_bounds__(tile::kThreads) void copy_convert_kernel(
     const void* __restrict__ src, int64_t ld_src, void* __restrict__ dst, int64_t ld_dst,
-    int64_t rows, int64_t cols, int vec_ok) {
+    int64_t rows, int64_t cols, int tpr_log2) {
   using namespace tile;
   constexpr int kSe = EltInfo<S>::bytes, kDe = EltInfo<D>::bytes;
   using SRaw = typename Raw8<kSe>::T;
   using DRaw = typename Raw8<kDe>::T;
-  for (int64_t r = blockIdx.y; r < rows; r += gridDim.y) {
-    const char* sp = (const char*)src + r * ld_src * kSe;
-    char* dp = (char*)dst + r * ld_dst * kDe;
-    SRaw in[kSlots];
-    // Loads first, conversions and stores after: kSlots loads in flight.
+  SRaw in[kSlots];
+  each_slot<WIDE>(
+      rows, cols, tpr_log2,
+      [&](int u, int64_t r, int64_t c) {
+        if (c + 8 <= cols) in[u] = load_any<SRaw>((const char*)src + (r * ld_src + c) * kSe);
+      },
+      [&](int u, int64_t r, int64_t c) {
+        if (c + 8 <= cols) {
+          float x[8];
 #pragma unroll
-    for (int u = 0; u < kSlots; ++u) {
-      const int64_t c = ((int64_t)(blockIdx.x * kSlots + u) * kThreads + threadIdx.x) * 8;
-      if (vec_ok && c + 8 <= cols) in[u] = *(const SRaw*)(sp + c * kSe);
-    }
-#pragma unroll
-    for (int u = 0; u < kSlots; ++u) {
-      const int64_t c = ((int64_t)(blockIdx.x * kSlots + u) * kThreads + threadIdx.x) * 8;
-      if (c >= cols) continue;
-      float x[8];
-      if (vec_ok && c + 8 <= cols) {
-#pragma unroll
-        for (int i = 0; i < 8; ++i) x[i] = elt_of<S>(&in[u], i);
-        DRaw out;
-        convert8<D>(x, &out);
-        *(DRaw*)(dp + c * kDe) = out;
-      } else {
-        for (int i = 0; i < 8 && c + i < cols; ++i) put<D>(dp, c + i, load_as_f32<S>(sp, c + i));
-      }
-    }
-  }
+          for (int i = 0; i < 8; ++i) x[i] = elt_of<S>(&in[u], i);
+          DRaw out;
+          convert8<D>(x, &out);
+          store_stream<DRaw>((char*)dst + (r * ld_dst + c) * kDe, out);
+        } else {
+          for (; c < cols; ++c) put<D>(dst, r * ld_dst + c, load_as_f32<S>(src, r * ld_src + c));
+        }
+      });
 }
 
-// Same-type copy of BYTES-wide elements (any dtype), same slot scheme.
+// An unsigned word of BYTES bytes.
 template <int BYTES>
+using WordOf = typename std::conditional<
+    BYTES == 1, uint8_t,
+    typename std::conditional<BYTES == 2, uint16_t,
+                              typename std::conditional<BYTES == 4, uint32_t, uint64_t>::type>::type>::type;
+
+// Same-type copy of BYTES-wide elements (any dtype).
+template <int BYTES, bool WIDE>
 __global__ __launch_bounds__(tile::kThreads) void copy_raw_kernel(
     const void* __restrict__ src, int64_t ld_src, void* __restrict__ dst, int64_t ld_dst,
-    int64_t rows, int64_t cols, int vec_ok) {
+    int64_t rows, int64_t cols, int tpr_log2) {
   using namespace tile;
   using Raw = typename Raw8<BYTES>::T;
-  using Word = typename std::conditional<
-      BYTES == 1, uint8_t,
-      typename std::conditional<BYTES == 2, uint16_t,
-                                typename std::conditional<BYTES == 4, uint32_t,
-                                                          uint64_t>::type>::type>::type;
-  for (int64_t r = blockIdx.y; r < rows; r += gridDim.y) {
-    const Word* sp = (const Word*)((const char*)src + r * ld_src * BYTES);
-    Word* dp = (Word*)((char*)dst + r * ld_dst * BYTES);
-    Raw in[kSlots];
-#pragma unroll
-    for (int u = 0; u < kSlots; ++u) {
-      const int64_t c = ((int64_t)(blockIdx.x * kSlots + u) * kThreads + threadIdx.x) * 8;
-      if (vec_ok && c + 8 <= cols) in[u] = *(const Raw*)(sp + c);
-    }
-#pragma unroll
-    for (int u = 0; u < kSlots; ++u) {
-      const int64_t c = ((int64_t)(blockIdx.x * kSlots + u) * kThreads + threadIdx.x) * 8;
-      if (c >= cols) continue;
-      if (vec_ok && c + 8 <= cols) {
-        *(Raw*)(dp + c) = in[u];
-      } else {
-        for (int i = 0; i < 8 && c + i < cols; ++i) dp[c + i] = sp[c + i];
-      }
-    }
-  }
+  using Word = WordOf<BYTES>;
+  const Word* sp = (const Word*)src;
+  Word* dp = (Word*)dst;
+  Raw in[kSlots];
+  each_slot<WIDE>(
+      rows, cols, tpr_log2,
+      [&](int u, int64_t r, int64_t c) {
+        if (c + 8 <= cols) in[u] = load_any<Raw>(sp + r * ld_src + c);
+      },
+      [&](int u, int64_t r, int64_t c) {
+        if (c + 8 <= cols) store_stream<Raw>(dp + r * ld_dst + c, in[u]);
+        else
+          for (; c < cols; ++c) dp[r * ld_dst + c] = sp[r * ld_src + c];
+      });
 }
 
-// Fill with a BYTES-wide bit pattern, same slot scheme.
-template <int BYTES>
+// Fill with a BYTES-wide bit pattern.
+template <int BYTES, bool WIDE>
 __global__ __launch_bounds__(tile::kThreads) void fill_kernel(void* __restrict__ dst, int64_t ld,
                                                               int64_t rows, int64_t cols,
-                                                              uint64_t bits, int vec_ok) {
+                                                              uint64_t bits, int tpr_log2) {
   using namespace tile;
   using Raw = typename Raw8<BYTES>::T;
-  using Word = typename std::conditional<
-      BYTES == 1, uint8_t,
-      typename std::conditional<BYTES == 2, uint16_t,
-                                typename std::conditional<BYTES == 4, uint32_t,
-                                                          uint64_t>::type>::type>::type;
+  using Word = WordOf<BYTES>;
+  Word* dp = (Word*)dst;
   Raw pat;
   Word* pw = (Word*)&pat;
 #pragma unroll
   for (int i = 0; i < 8; ++i) pw[i] = (Word)bits;
-  for (int64_t r = blockIdx.y; r < rows; r += gridDim.y) {
-    Word* dp = (Word*)((char*)dst + r * ld * BYTES);
-#pragma unroll
-    for (int u = 0; u < kSlots; ++u) {
-      const int64_t c = ((int64_t)(blockIdx.x * kSlots + u) * kThreads + threadIdx.x) * 8;
-      if (c >= cols) continue;
-      if (vec_ok && c + 8 <= cols) {
-        *(Raw*)(dp + c) = pat;
-      } else {
-        for (int i = 0; i < 8 && c + i < cols; ++i) dp[c + i] = (Word)bits;
-      }
-    }
-  }
+  each_slot<WIDE>(
+      rows, cols, tpr_log2, [](int, int64_t, int64_t) {},
+      [&](int, int64_t r, int64_t c) {
+        if (c + 8 <= cols) store_any<Raw>(dp + r * ld + c, pat);
+        else
+          for (; c < cols; ++c) dp[r * ld + c] = (Word)bits;
+      });
 }
 
 // ---- launchers ------------------------------------------------------------------------
@@ -604,10 +565,6 @@ int ilog2(int64_t x) {
   int l = 0;
   while (((int64_t)1 << l) < x) ++l;
   return l;
-}
-
-bool aligned(const void* p, int64_t ld_bytes, int a) {
-  return ((uintptr_t)p % a) == 0 && ld_bytes % a == 0;
 }
 
 }  // namespace
@@ -634,6 +591,34 @@ ColsSplit cols_split(int64_t rows, int64_t cols) {
 
 namespace {
 
+// One pass over `rows` rows of src (of a.cols columns) into a.dst.
+template <Elt E, Elt LOAD, int KIND, int T>
+hipError_t cols_pass(const void* src, int64_t ld, int64_t rows, const ReduceArgs& a, float* partial,
+                     hipStream_t s) {
+  const int64_t slots = (a.cols + 3) / 4;
+  // The widest strips, up to 64 slots, that still give a workgroup per CU (at
+  // least 8 slots, 128 bytes of f32); and no more row groups than runs of
+  // eight rows.
+  int cvb_log2 = 6;
+  while (cvb_log2 > 3 && (slots + (1 << cvb_log2) - 1) >> cvb_log2 < 256) --cvb_log2;
+  const int t_log2 = ilog2(T), runs = ilog2((rows + 7) / 8);
+  if (t_log2 - cvb_log2 > runs) cvb_log2 = t_log2 - runs;
+  const int groups_log2 = t_log2 - cvb_log2;
+  int b_log2 = ilog2((rows + ((int64_t)1 << groups_log2) - 1) >> groups_log2);
+  if (b_log2 < 3) b_log2 = 3;
+  const dim3 grid((unsigned)((slots + ((int64_t)1 << cvb_log2) - 1) >> cvb_log2));
+#define FRISK_COLS(LV)                                                                           \
+  hipLaunchKernelGGL((reduce_cols_kernel<E, LOAD, KIND, T, LV>), grid, dim3(T), 0, s, src, ld, rows, \
+                     a.cols, a.dst, a.dst_stride, a.clear, cvb_log2, b_log2, partial)
+  // 2^(b_log2 - 3) pushes fill up to b_log2 - 2 levels of a sum's counter;
+  // with more than 6 of them (4 columns each) 1024 threads have no registers.
+  if (KIND != kReduceSum || b_log2 <= 8) FRISK_COLS(6);
+  else if constexpr (T > 256) return cols_pass<E, LOAD, KIND, 256>(src, ld, rows, a, partial, s);
+  else FRISK_COLS(22);
+#undef FRISK_COLS
+  return hipGetLastError();
+}
+
 template <Elt E, int KIND>
 hipError_t reduce_typed(const ReduceArgs& a, hipStream_t s) {
   constexpr int kEsz = EltInfo<E>::bytes;
@@ -651,53 +636,60 @@ hipError_t reduce_typed(const ReduceArgs& a, hipStream_t s) {
     const int64_t slots = (a.cols + V - 1) / V;
     const int pl = ilog2(slots);  // log2 of the padded slot count
     const int lpr_log2 = pl < 6 ? pl : 6;
-    const int r_log2 = pl - 6 > 3 ? 3 : (pl > 6 ? pl - 6 : 0);
+    // Waves per row: enough for 2048 waves (8 per CU) as long as a row has 64
+    // slots for each.
+    int wpr_log2 = 0;
+    while (wpr_log2 < 4 && (a.rows << wpr_log2) < 2048 && pl - 6 > wpr_log2 + 1) wpr_log2 += 2;
+    const int left = pl - 6 - wpr_log2;
+    const int r_log2 = left > 3 ? 3 : left > 0 ? left : 0;
     const int64_t S = ((int64_t)1 << (lpr_log2 + r_log2)) * V;
     const uint32_t chunks = (uint32_t)((a.cols + S - 1) / S);
-    const int vec_ok = aligned(a.src, a.ld * kEsz, 16);
+    const uint32_t per_wave = 1u << ilog2((chunks + (1u << wpr_log2) - 1) >> wpr_log2);
     const int64_t rows_per_block = (int64_t)(tile::kThreads / 64) << (6 - lpr_log2);
-    const dim3 grid((unsigned)((a.rows + rows_per_block - 1) / rows_per_block));
-#define FRISK_ROWS(R)                                                                        \
-  hipLaunchKernelGGL((reduce_rows_kernel<E, KIND, R>), grid, dim3(tile::kThreads), 0, s, a.src, \
-                     a.ld, a.rows, a.cols, a.dst, a.dst_stride, a.clear, lpr_log2, vec_ok, chunks)
-    switch (r_log2) {
-      case 0: FRISK_ROWS(1); break;
-      case 1: FRISK_ROWS(2); break;
-      case 2: FRISK_ROWS(4); break;
-      default: FRISK_ROWS(8); break;
-    }
-#undef FRISK_ROWS
-  } else if (a.workspace) {
-    const ColsSplit sp = cols_split(a.rows, a.cols);
-    const int vec_ok = aligned(a.src, a.ld * kEsz, 4 * kEsz);
-    hipLaunchKernelGGL((reduce_cols_blocks_kernel<E, KIND>), dim3(sp.strips, sp.blocks),
-                       dim3(tile::kThreads), 0, s, a.src, a.ld, a.rows, a.cols, sp.sps_log2,
-                       sp.b_log2, (float*)a.workspace, vec_ok);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL((reduce_cols_final_kernel<E, KIND>),
-                       dim3((unsigned)((a.cols + tile::kThreads - 1) / tile::kThreads)),
-                       dim3(tile::kThreads), 0, s, (const float*)a.workspace, a.cols,
-                       (uint32_t)sp.blocks, a.dst, a.dst_stride, a.clear);
-  } else {
-    const int64_t slots = (a.cols + 3) / 4;
-    // Widest column strip (best coalescing) that still yields >= 1024
-    // workgroups; at least 8 slots (128 B of f32 per row) when there are
-    // that many columns.
-    int cvb_log2 = 6;
-    while (cvb_log2 > 3 && (slots + (1 << cvb_log2) - 1) >> cvb_log2 < 1024) --cvb_log2;
-    const int pl = ilog2(slots);
-    if (pl < cvb_log2) cvb_log2 = pl;
-    const int groups = kColThreads >> cvb_log2;
-    int b_log2 = ilog2((a.rows + groups - 1) / groups);
-    if (b_log2 < 3) b_log2 = 3;
-    const int vec_ok = aligned(a.src, a.ld * kEsz, 4 * kEsz);
-    const dim3 grid((unsigned)((slots + (1 << cvb_log2) - 1) >> cvb_log2));
-    hipLaunchKernelGGL((reduce_cols_kernel<E, KIND>), grid, dim3(kColThreads), 0, s, a.src,
-                       a.ld, a.rows, a.cols, a.dst, a.dst_stride, a.clear, cvb_log2, b_log2,
-                       vec_ok);
+    const dim3 grid((unsigned)(wpr_log2 ? a.rows : (a.rows + rows_per_block - 1) / rows_per_block));
+#define FRISK_ROWS(R, W)                                                                       \
+  hipLaunchKernelGGL((reduce_rows_kernel<E, KIND, R, W>), grid,                                \
+                     dim3(W > 4 ? 64 * W : tile::kThreads), 0, s, a.src, a.ld, a.rows, a.cols, \
+                     a.dst, a.dst_stride, a.clear, lpr_log2, chunks, per_wave)
+#define FRISK_ROWS_R(W)             \
+  switch (r_log2) {                 \
+    case 0: FRISK_ROWS(1, W); break; \
+    case 1: FRISK_ROWS(2, W); break; \
+    case 2: FRISK_ROWS(4, W); break; \
+    default: FRISK_ROWS(8, W);       \
   }
-  return hipGetLastError();
+    if (wpr_log2 == 0) FRISK_ROWS_R(1)
+    else if (wpr_log2 == 2) FRISK_ROWS_R(4)
+    else FRISK_ROWS_R(16)
+#undef FRISK_ROWS_R
+#undef FRISK_ROWS
+    return hipGetLastError();
+  }
+  const int64_t slots = (a.cols + 3) / 4;
+  // One pass of 1024-thread workgroups when strips of 16 slots (256 bytes of
+  // an f32 row) give at least 200 of them, or where there is no workspace;
+  // under 256 rows 256 threads.  Two passes otherwise, through f32 partials.
+  // One against two passes, us: f32 8192x16384 92.9 and 90.6, 4096x32768 96.4
+  // and 99.2, 2048x16384 25.3 and 27.3, 300x14000 8.3 and 12.1, bf16
+  // 1024x65536 26.8 and 31.5.  (Before, two passes from 256 rows on and below
+  // them 1024 threads a strip, most without rows: max 125, 125, 41.5, 16.5 and
+  // 68 f32; 112x15874 23.6 -> 6.8; 17920x128, whose second pass walked 280
+  // partials in one workgroup, 49.3 -> 11.3.)
+  if (a.rows < 256) return cols_pass<E, E, KIND, 256>(a.src, a.ld, a.rows, a, nullptr, s);
+  if (!a.workspace || (slots >= 200 * 16))
+    return cols_pass<E, E, KIND, 1024>(a.src, a.ld, a.rows, a, nullptr, s);
+  const ColsSplit sp = cols_split(a.rows, a.cols);
+  const int run_log2 = sp.b_log2 - (8 - sp.sps_log2);  // rows a group: at most 2^12, 10 levels
+#define FRISK_BLOCKS(LV)                                                                             \
+  hipLaunchKernelGGL((reduce_cols_kernel<E, E, KIND, 256, LV>), dim3(sp.strips, sp.blocks), dim3(256), \
+                     0, s, a.src, a.ld, a.rows, a.cols, a.dst, a.dst_stride, a.clear, sp.sps_log2,    \
+                     run_log2, (float*)a.workspace)
+  if (KIND != kReduceSum || run_log2 <= 8) FRISK_BLOCKS(6);
+  else FRISK_BLOCKS(10);
+#undef FRISK_BLOCKS
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  return cols_pass<E, Elt::F32, KIND, 256>(a.workspace, a.cols, sp.blocks, a, nullptr, s);
 }
 
 template <Elt E>
@@ -710,20 +702,30 @@ hipError_t reduce_kind(const ReduceArgs& a, hipStream_t s) {
   }
 }
 
-dim3 slot_grid(int64_t rows, int64_t cols) {
-  const int64_t per_block = (int64_t)tile::kThreads * tile::kSlots * 8;
-  return dim3((unsigned)((cols + per_block - 1) / per_block),
-              (unsigned)(rows < 65535 ? rows : 65535));
+// Grid and threads per row of each_slot.
+struct SlotGrid {
+  dim3 grid;
+  int tpr_log2;
+};
+SlotGrid slot_grid(int64_t rows, int64_t cols) {
+  const int64_t slots = (cols + 7) / 8;
+  if (slots > tile::kThreads / 2) {
+    const int64_t per_block = (int64_t)tile::kThreads * tile::kSlots * 8;
+    return SlotGrid{dim3((unsigned)((cols + per_block - 1) / per_block),
+                         (unsigned)(rows < 65535 ? rows : 65535)), -1};
+  }
+  const int tpr_log2 = ilog2(slots);
+  const int64_t per_block = (int64_t)(tile::kThreads >> tpr_log2) * tile::kSlots;
+  const int64_t blocks = (rows + per_block - 1) / per_block;
+  return SlotGrid{dim3((unsigned)(blocks < (1 << 20) ? blocks : 1 << 20)), tpr_log2};
 }
 
 template <Elt S, Elt D>
 hipError_t copy_typed(const CopyArgs& a, hipStream_t s) {
-  constexpr int kSe = EltInfo<S>::bytes, kDe = EltInfo<D>::bytes;
-  const int vec_ok = aligned(a.src, a.ld_src * kSe, 8 * kSe < 16 ? 8 * kSe : 16) &&
-                     aligned(a.dst, a.ld_dst * kDe, 8 * kDe < 16 ? 8 * kDe : 16);
-  hipLaunchKernelGGL((copy_convert_kernel<S, D>), slot_grid(a.rows, a.cols),
-                     dim3(tile::kThreads), 0, s, a.src, a.ld_src, a.dst, a.ld_dst, a.rows, a.cols,
-                     vec_ok);
+  const SlotGrid g = slot_grid(a.rows, a.cols);
+  auto kern = g.tpr_log2 < 0 ? copy_convert_kernel<S, D, true> : copy_convert_kernel<S, D, false>;
+  hipLaunchKernelGGL(kern, g.grid, dim3(tile::kThreads), 0, s, a.src, a.ld_src,
+                     a.dst, a.ld_dst, a.rows, a.cols, g.tpr_log2);
   return hipGetLastError();
 }
 
@@ -740,19 +742,19 @@ hipError_t copy_from(const CopyArgs& a, hipStream_t s) {
 
 template <int BYTES>
 hipError_t copy_raw(const CopyArgs& a, hipStream_t s) {
-  const int va = 8 * BYTES < 16 ? 8 * BYTES : 16;
-  const int vec_ok = aligned(a.src, a.ld_src * BYTES, va) && aligned(a.dst, a.ld_dst * BYTES, va);
-  hipLaunchKernelGGL((copy_raw_kernel<BYTES>), slot_grid(a.rows, a.cols), dim3(tile::kThreads), 0,
-                     s, a.src, a.ld_src, a.dst, a.ld_dst, a.rows, a.cols, vec_ok);
+  const SlotGrid g = slot_grid(a.rows, a.cols);
+  auto kern = g.tpr_log2 < 0 ? copy_raw_kernel<BYTES, true> : copy_raw_kernel<BYTES, false>;
+  hipLaunchKernelGGL(kern, g.grid, dim3(tile::kThreads), 0, s, a.src, a.ld_src,
+                     a.dst, a.ld_dst, a.rows, a.cols, g.tpr_log2);
   return hipGetLastError();
 }
 
 template <int BYTES>
 hipError_t fill_bytes(const FillArgs& a, hipStream_t s) {
-  const int va = 8 * BYTES < 16 ? 8 * BYTES : 16;
-  const int vec_ok = aligned(a.dst, a.ld * BYTES, va);
-  hipLaunchKernelGGL((fill_kernel<BYTES>), slot_grid(a.rows, a.cols), dim3(tile::kThreads), 0, s,
-                     a.dst, a.ld, a.rows, a.cols, a.bits, vec_ok);
+  const SlotGrid g = slot_grid(a.rows, a.cols);
+  auto kern = g.tpr_log2 < 0 ? fill_kernel<BYTES, true> : fill_kernel<BYTES, false>;
+  hipLaunchKernelGGL(kern, g.grid, dim3(tile::kThreads), 0, s, a.dst, a.ld, a.rows,
+                     a.cols, a.bits, g.tpr_log2);
   return hipGetLastError();
 }
 
