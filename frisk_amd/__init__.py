@@ -72,7 +72,15 @@ def __getattr__(name: str):
         return parse_module
     if name.startswith("__") or name == "frisk_ffi":
         raise AttributeError(name)
-    ir = _ir()
+    try:
+        ir = _ir()
+    except ImportError:
+        # `from frisk_amd import build` asks here first; an AttributeError
+        # makes the import system load the submodule.
+        from importlib.util import find_spec
+        if find_spec(f"{__name__}.{name}") is not None:
+            raise AttributeError(name) from None
+        raise
     if hasattr(ir, name):
         return getattr(ir, name)
     raise AttributeError(f"module 'frisk_amd' has no attribute '{name}'")
