@@ -181,6 +181,19 @@ def _stream_handle(stream) -> int:
     return int(stream.cuda_stream) if hasattr(stream, "cuda_stream") else int(stream)
 
 
+def _scratch(nbytes: int, device, stream):
+    """A call's scratch, allocated on the stream its kernels run on: the
+    allocator may hand it out again as soon as it is dropped, to work of that
+    stream only."""
+    import torch
+    if stream is None:
+        return torch.empty(nbytes, dtype=torch.uint8, device=device)
+    if not hasattr(stream, "cuda_stream"):
+        stream = torch.cuda.ExternalStream(int(stream), device=device)
+    with torch.cuda.stream(stream):
+        return torch.empty(nbytes, dtype=torch.uint8, device=device)
+
+
 def _row_major(t, name: str) -> int:
     if t.dim() != 2 or t.stride(1) != 1:
         raise ValueError(f"{name} must be a rank-2 tensor with unit column stride")
@@ -258,9 +271,7 @@ def gemm(a, b, c, *, trans_a=False, trans_b=False, clear_accum=True,
         need = load().frisk_gemm_workspace_size(ctypes.byref(d))
         _check(int(need) if need < 0 else OK, "frisk_gemm_workspace_size")
         if need > 0:
-            import torch
-            ws = workspace if workspace is not True else \
-                torch.empty(need, dtype=torch.uint8, device=c.device)
+            ws = workspace if workspace is not True else _scratch(need, c.device, stream)
             d.workspace, d.workspace_bytes = ws.data_ptr(), ws.numel() * ws.element_size()
     _check(load().frisk_gemm(ctypes.byref(d), ctypes.c_void_p(_stream_handle(stream))),
            "frisk_gemm")
@@ -366,8 +377,7 @@ def attn_fwd(q, k, v, o, *, causal=False, sm_scale=None, lse=None, stream=None,
         need = lib.frisk_attn_workspace_size(ctypes.byref(d))
         _check(int(need) if need < 0 else OK, "frisk_attn_fwd")
     if need > 0:
-        import torch
-        ws = torch.empty(need, dtype=torch.uint8, device=o.device)
+        ws = _scratch(need, o.device, stream)
         rc = lib.frisk_attn_fwd_ws(ctypes.byref(d), ws.data_ptr(), need,
                                    ctypes.c_void_p(_stream_handle(stream)))
     else:
@@ -433,9 +443,7 @@ def reduce(src, dst, kind="sum", *, axis=1, clear=True, leaf_order=None, workspa
         need = load().frisk_reduce_workspace_size(ctypes.byref(d))
         _check(int(need) if need < 0 else OK, "frisk_reduce_workspace_size")
         if need > 0:
-            import torch
-            ws = workspace if workspace is not True else \
-                torch.empty(need, dtype=torch.uint8, device=src.device)
+            ws = workspace if workspace is not True else _scratch(need, src.device, stream)
             d.workspace, d.workspace_bytes = ws.data_ptr(), ws.numel() * ws.element_size()
     _check(load().frisk_reduce(ctypes.byref(d), ctypes.c_void_p(_stream_handle(stream))),
            "frisk_reduce")

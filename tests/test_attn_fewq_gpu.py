@@ -88,3 +88,36 @@ def test_few_queries_repeat_bitwise_and_through_the_binding():
     ref, _ = A.attention_fp64(q.double().cpu().numpy(), k.double().cpu().numpy(),
                               v.double().cpu().numpy(), causal=True, scale=128 ** -0.5)
     assert G.row_scaled_error(outs[0].double().cpu().numpy(), ref) <= 1e-2
+
+
+@pytest.mark.parametrize("as_handle", [False, True])
+def test_scratch_belongs_to_the_stream_of_the_call(monkeypatch, as_handle):
+    """On another stream than the current one, the scratch of a call comes
+    from that stream's pool: a tensor of the current stream never reuses it
+    while the kernels run."""
+    side = torch.cuda.Stream()
+    stream = side.cuda_stream if as_handle else side
+    seen, empty = [], torch.empty
+
+    def recorded(*a, **kw):
+        seen.append(torch.cuda.current_stream().cuda_stream)
+        return empty(*a, **kw)
+
+    g = gen(5)
+    q = torch.randn(1, 1, 1, 128, generator=g, device="cuda").to(torch.bfloat16)
+    k, v = (torch.randn(1, 1, 4096, 128, generator=g, device="cuda").to(torch.bfloat16) for _ in range(2))
+    a = torch.randn(2, 13418, generator=g, device="cuda").to(torch.bfloat16)
+    b = torch.randn(13418, 210, generator=g, device="cuda").to(torch.bfloat16)
+    x = torch.randn(8192, 1024, generator=g, device="cuda")
+    outs = [torch.zeros_like(q), torch.zeros(2, 210, device="cuda"), torch.zeros(1024, device="cuda")]
+    calls = [lambda o, **kw: rt.attn_fwd(q, k, v, o, **kw), lambda o, **kw: rt.gemm(a, b, o, **kw),
+             lambda o, **kw: rt.reduce(x, o, "max", axis=0, **kw)]
+    ref = [call_(torch.zeros_like(o)) for call_, o in zip(calls, outs)]
+    torch.cuda.synchronize()
+    monkeypatch.setattr(torch, "empty", recorded)
+    for call_, o in zip(calls, outs):
+        call_(o, stream=stream)
+    monkeypatch.undo()
+    torch.cuda.synchronize()
+    assert seen == [side.cuda_stream] * 3
+    assert all(torch.equal(o, r) for o, r in zip(outs, ref))
