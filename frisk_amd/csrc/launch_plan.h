@@ -543,5 +543,57 @@ inline int64_t attn_workspace(int64_t batch_heads, int64_t seq_q, int64_t seq_k,
   return s > 1 ? batch_heads * s * seq_q * (head_dim + 2) * 4 : 0;
 }
 
+// ---------------------------------------------------------------------------
+// Reductions along axis 0 (tileops.hip), of [rows, cols] in slots of 4 columns.
+//
+// One pass: a workgroup of `threads` owns a strip of 2^cvb_log2 slots; its
+// threads >> cvb_log2 row groups each walk runs of 2^b_log2 rows.  The strips
+// are the widest, up to 64 slots, that still give a workgroup per CU (at
+// least 8 slots, 128 bytes of f32, of the slots there are), and no workgroup
+// has more row groups than runs of eight rows.  1024 threads, since the grid
+// has one workgroup per strip only; under 256 rows 256 threads.
+//
+// A sum's counter holds a level per doubling of the run, and 1024 threads have
+// registers for 6 of them (4 columns each): runs of 256 rows.  A longer sum
+// takes the rows in `blocks` blocks of groups x 256, whose roots combine in
+// LDS; or, where the strips fill the CUs in whole rounds, runs in 256 threads
+// a strip with a counter of 22 levels in registers.  us, f32 sum without a
+// workspace, 256 threads and 1024 in blocks: 300000x64 1369, 711; 50000x4000
+// 212, 158; 65536x12800 752, 679; 16384x32768 301, 376; 32768x16384 309, 390.
+// (100000x3, whose strip is held to the one slot there is: 150; as 8 slots on
+// 32 live threads of 256, 489.)
+// ---------------------------------------------------------------------------
+struct ColsPass {
+  int threads, cvb_log2, b_log2, blocks;
+  int64_t strips;
+};
+
+inline int ilog2_ceil(int64_t x) {
+  int l = 0;
+  while (((int64_t)1 << l) < x) ++l;
+  return l;
+}
+
+// The strips occupy at least nine tenths of the CU rounds they take.
+inline bool strips_fill(int64_t strips) { return strips * 10 >= rounds(strips, 256) * 256 * 9; }
+
+inline ColsPass cols_pass(int64_t rows, int64_t cols, bool sum, int threads) {
+  ColsPass p{threads, 6, 0, 1, 0};
+  const int64_t slots = (cols + 3) / 4;
+  while (p.cvb_log2 > 3 && (slots + (1 << p.cvb_log2) - 1) >> p.cvb_log2 < 256) --p.cvb_log2;
+  p.cvb_log2 = std::min(p.cvb_log2, ilog2_ceil(slots));
+  const int runs = ilog2_ceil((rows + 7) / 8);
+  p.cvb_log2 = std::max(p.cvb_log2, ilog2_ceil(threads) - runs);
+  p.strips = (slots + ((int64_t)1 << p.cvb_log2) - 1) >> p.cvb_log2;
+  const int groups_log2 = ilog2_ceil(threads) - p.cvb_log2;
+  p.b_log2 = std::max(3, ilog2_ceil((rows + ((int64_t)1 << groups_log2) - 1) >> groups_log2));
+  if (sum && p.b_log2 > 8 && threads > 256) {
+    if (p.strips >= 256 && strips_fill(p.strips)) return cols_pass(rows, cols, sum, 256);
+    p.b_log2 = 8;
+    p.blocks = (int)((rows + ((int64_t)1 << (groups_log2 + 8)) - 1) >> (groups_log2 + 8));
+  }
+  return p;
+}
+
 }  // namespace plan
 }  // namespace frisk

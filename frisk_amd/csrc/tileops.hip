@@ -230,84 +230,99 @@ __global__ __launch_bounds__(WPR > 4 ? 64 * WPR : tile::kThreads) void reduce_ro
 
 // ---- axis 0: reduce across rows -------------------------------------------------
 // A workgroup of T threads owns 2^cvb_log2 slots of 4 adjacent columns and the
-// rows [block B, (block + 1) B) of its blockIdx.y; its T >> cvb_log2 row groups
-// each take an aligned run of 2^b_log2 (>= 8) of them.  A thread walks its run
-// eight rows at a time: the eight-row subtree is built in registers and pushed
-// into a binary counter of LV levels.  The groups' roots (complete subtrees;
-// an empty run is the identity) are combined in LDS by the pairwise tree over
-// the groups, and go to dst, or, in the first of two passes, to
-// partial[block][column] as f32; the second pass is the same kernel over the
-// partials (LOAD f32) with the combines of E.
-template <Elt E, Elt LOAD, int KIND, int T, int LV>
+// rows of block blockIdx.y, or with TOP all `blocks` blocks one after another;
+// in a block its T >> cvb_log2 row groups each take an aligned run of 2^b_log2
+// (>= 8) rows.  A thread walks its run eight rows at a time: the eight-row
+// subtree is built in registers and pushed into a binary counter of LV levels.
+// The groups' roots (complete subtrees; an empty run is the identity) are
+// combined in LDS by the pairwise tree over the groups.  The block's root goes
+// to dst, or, in the first of two passes, to partial[block][column] as f32
+// (the second pass is the same kernel over the partials, LOAD f32, with the
+// combines of E), or, with TOP, into a binary counter of TOP levels in LDS.
+template <Elt E, Elt LOAD, int KIND, int T, int LV, int TOP>
 __global__ __launch_bounds__(T, T > 256 || LV <= 6 ? 4 : 1) void reduce_cols_kernel(
     const void* __restrict__ src, int64_t ld, int64_t rows, int64_t cols, void* __restrict__ dst,
-    int64_t dst_stride, int clear, int cvb_log2, int b_log2, float* __restrict__ partial) {
+    int64_t dst_stride, int clear, int cvb_log2, int b_log2, int blocks, float* __restrict__ partial) {
   using namespace tile;
   constexpr int kEsz = EltInfo<LOAD>::bytes;
   __shared__ float part[T * 4];
+  __shared__ float top[TOP > 0 ? TOP * 256 : 1];
   const int tid = threadIdx.x;
   const int cvb = 1 << cvb_log2;
   const int cs = tid & (cvb - 1), g = tid >> cvb_log2;
   const int groups = T >> cvb_log2;
   const int64_t c0 = ((int64_t)blockIdx.x * cvb + cs) * 4;
-  const int64_t r0 = ((int64_t)blockIdx.y * groups + g) << b_log2;
-  const int64_t r1 = min(rows, r0 + ((int64_t)1 << b_log2));
   const bool full = c0 + 4 <= cols;
 
-  Counter<E, KIND, LV, 4> ctr;
-  uint32_t n8 = 0;
-  for (int64_t i0 = r0; i0 < r1; i0 += 8, ++n8) {
-    float x[8][4];
-    const char* rp = (const char*)src + (i0 * ld + c0) * kEsz;
-    if (full && i0 + 8 <= r1) {
+  for (int k = 0; k < (TOP > 0 ? blocks : 1); ++k) {
+    const int64_t r0 = ((int64_t)(blockIdx.y + k) * groups + g) << b_log2;
+    const int64_t r1 = min(rows, r0 + ((int64_t)1 << b_log2));
+    Counter<E, KIND, LV, 4> ctr;
+    uint32_t n8 = 0;
+    for (int64_t i0 = r0; i0 < r1; i0 += 8, ++n8) {
+      float x[8][4];
+      const char* rp = (const char*)src + (i0 * ld + c0) * kEsz;
+      if (full && i0 + 8 <= r1) {
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const char* p = rp + i * ld * kEsz;
-        if constexpr (LOAD == Elt::F32) {
-          const f32x4 v = __builtin_nontemporal_load((const f32x4_any*)p);
+        for (int i = 0; i < 8; ++i) {
+          const char* p = rp + i * ld * kEsz;
+          if constexpr (LOAD == Elt::F32) {
+            const f32x4 v = __builtin_nontemporal_load((const f32x4_any*)p);
 #pragma unroll
-          for (int j = 0; j < 4; ++j) x[i][j] = v[j];
-        } else {
-          const i32x2 v = __builtin_nontemporal_load((const i32x2_any*)p);
+            for (int j = 0; j < 4; ++j) x[i][j] = v[j];
+          } else {
+            const i32x2 v = __builtin_nontemporal_load((const i32x2_any*)p);
 #pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            const uint16_t h = (uint16_t)((uint32_t)v[j >> 1] >> (16 * (j & 1)));
-            x[i][j] = LOAD == Elt::BF16 ? bf16_bits_to_f32(h) : (float)__builtin_bit_cast(_Float16, h);
+            for (int j = 0; j < 4; ++j) {
+              const uint16_t h = (uint16_t)((uint32_t)v[j >> 1] >> (16 * (j & 1)));
+              x[i][j] = LOAD == Elt::BF16 ? bf16_bits_to_f32(h) : (float)__builtin_bit_cast(_Float16, h);
+            }
           }
         }
-      }
-    } else {
+      } else {
 #pragma unroll
-      for (int i = 0; i < 8; ++i)
+        for (int i = 0; i < 8; ++i)
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+            x[i][j] = i0 + i < r1 && c0 + j < cols ? load_as_f32<LOAD>(rp + i * ld * kEsz, j)
+                                                   : identity<KIND>();
+      }
+      float t[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+#pragma unroll
+        for (int w = 1; w < 8; w <<= 1)
+#pragma unroll
+          for (int i = 0; i < 8; i += 2 * w) x[i][j] = combine<E, KIND>(x[i][j], x[i + w][j]);
+        t[j] = x[0][j];
+      }
+      ctr.push(n8, t);
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) part[(g * cvb + cs) * 4 + j] = ctr.finish(n8, j);
+    __syncthreads();
+    // The pairwise tree over the row groups, one level at a time across the
+    // workgroup: at level w group g (a multiple of 2w) takes in group g + w.
+    for (int w = 1; w < groups; w <<= 1) {
+      if ((g & (2 * w - 1)) == 0) {
 #pragma unroll
         for (int j = 0; j < 4; ++j)
-          x[i][j] = i0 + i < r1 && c0 + j < cols ? load_as_f32<LOAD>(rp + i * ld * kEsz, j)
-                                                 : identity<KIND>();
+          part[(g * cvb + cs) * 4 + j] = combine<E, KIND>(part[(g * cvb + cs) * 4 + j],
+                                                          part[((g + w) * cvb + cs) * 4 + j]);
+      }
+      __syncthreads();
     }
-    float t[4];
+    // (Only the thread of its columns touches an entry of `top`, and part of
+    // group 0.)
+    if (TOP > 0 && g == 0) {
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-#pragma unroll
-      for (int w = 1; w < 8; w <<= 1)
-#pragma unroll
-        for (int i = 0; i < 8; i += 2 * w) x[i][j] = combine<E, KIND>(x[i][j], x[i + w][j]);
-      t[j] = x[0][j];
+      for (int j = 0; j < 4; ++j) {
+        float x = part[cs * 4 + j];
+        int l = 0;
+        for (; (k >> l) & 1; ++l) x = combine<E, KIND>(top[l * 256 + cs * 4 + j], x);
+        top[l * 256 + cs * 4 + j] = x;
+      }
     }
-    ctr.push(n8, t);
-  }
-#pragma unroll
-  for (int j = 0; j < 4; ++j) part[(g * cvb + cs) * 4 + j] = ctr.finish(n8, j);
-  __syncthreads();
-  // The pairwise tree over the row groups, one level at a time across the
-  // workgroup: at level w group g (a multiple of 2w) takes in group g + w.
-  for (int w = 1; w < groups; w <<= 1) {
-    if ((g & (2 * w - 1)) == 0) {
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-        part[(g * cvb + cs) * 4 + j] = combine<E, KIND>(part[(g * cvb + cs) * 4 + j],
-                                                        part[((g + w) * cvb + cs) * 4 + j]);
-    }
-    __syncthreads();
   }
   if (g == 0) {
 #pragma unroll
@@ -315,6 +330,12 @@ __global__ __launch_bounds__(T, T > 256 || LV <= 6 ? 4 : 1) void reduce_cols_ker
       const int64_t c = c0 + j;
       if (c < cols) {
         float res = part[cs * 4 + j];
+        if constexpr (TOP > 0) {  // from the smallest (rightmost) set of blocks up
+          int l = __builtin_ctz(blocks);
+          res = top[l * 256 + cs * 4 + j];
+          for (++l; blocks >> l; ++l)
+            if ((blocks >> l) & 1) res = combine<E, KIND>(top[l * 256 + cs * 4 + j], res);
+        }
         if (partial) {
           partial[(int64_t)blockIdx.y * cols + c] = res;
         } else {
@@ -591,30 +612,25 @@ ColsSplit cols_split(int64_t rows, int64_t cols) {
 
 namespace {
 
-// One pass over `rows` rows of src (of a.cols columns) into a.dst.
+// One pass over `rows` rows of src (of a.cols columns) into a.dst
+// (plan::cols_pass).  T 256: at most 256 * 2^8 rows of a sum's few partials.
 template <Elt E, Elt LOAD, int KIND, int T>
-hipError_t cols_pass(const void* src, int64_t ld, int64_t rows, const ReduceArgs& a, float* partial,
-                     hipStream_t s) {
-  const int64_t slots = (a.cols + 3) / 4;
-  // The widest strips, up to 64 slots, that still give a workgroup per CU (at
-  // least 8 slots, 128 bytes of f32); and no more row groups than runs of
-  // eight rows.
-  int cvb_log2 = 6;
-  while (cvb_log2 > 3 && (slots + (1 << cvb_log2) - 1) >> cvb_log2 < 256) --cvb_log2;
-  const int t_log2 = ilog2(T), runs = ilog2((rows + 7) / 8);
-  if (t_log2 - cvb_log2 > runs) cvb_log2 = t_log2 - runs;
-  const int groups_log2 = t_log2 - cvb_log2;
-  int b_log2 = ilog2((rows + ((int64_t)1 << groups_log2) - 1) >> groups_log2);
-  if (b_log2 < 3) b_log2 = 3;
-  const dim3 grid((unsigned)((slots + ((int64_t)1 << cvb_log2) - 1) >> cvb_log2));
-#define FRISK_COLS(LV)                                                                           \
-  hipLaunchKernelGGL((reduce_cols_kernel<E, LOAD, KIND, T, LV>), grid, dim3(T), 0, s, src, ld, rows, \
-                     a.cols, a.dst, a.dst_stride, a.clear, cvb_log2, b_log2, partial)
-  // 2^(b_log2 - 3) pushes fill up to b_log2 - 2 levels of a sum's counter;
-  // with more than 6 of them (4 columns each) 1024 threads have no registers.
-  if (KIND != kReduceSum || b_log2 <= 8) FRISK_COLS(6);
-  else if constexpr (T > 256) return cols_pass<E, LOAD, KIND, 256>(src, ld, rows, a, partial, s);
-  else FRISK_COLS(22);
+hipError_t cols_pass(const void* src, int64_t ld, int64_t rows, const ReduceArgs& a, hipStream_t s) {
+  const plan::ColsPass p = plan::cols_pass(rows, a.cols, KIND == kReduceSum, T);
+#define FRISK_COLS(THREADS, LV, TOP)                                                                \
+  hipLaunchKernelGGL((reduce_cols_kernel<E, LOAD, KIND, THREADS, LV, TOP>), dim3((unsigned)p.strips), \
+                     dim3(THREADS), 0, s, src, ld, rows, a.cols, a.dst, a.dst_stride, a.clear,      \
+                     p.cvb_log2, p.b_log2, p.blocks, (float*)nullptr)
+  // A run of 2^b_log2 rows is 2^(b_log2 - 3) pushes, which fill up to
+  // b_log2 - 2 levels; rows < 2^23 in blocks of at least 2^12 fill 12.
+  if constexpr (KIND == kReduceSum && T > 256) {
+    if (p.blocks > 1) FRISK_COLS(T, 6, 12);
+    else if (p.b_log2 > 8) FRISK_COLS(256, 22, 0);
+    else FRISK_COLS(T, 6, 0);
+  } else {
+    if (KIND == kReduceSum && p.b_log2 > 8) return hipErrorInvalidValue;  // no such call
+    FRISK_COLS(T, 6, 0);
+  }
 #undef FRISK_COLS
   return hipGetLastError();
 }
@@ -675,21 +691,21 @@ hipError_t reduce_typed(const ReduceArgs& a, hipStream_t s) {
   // them 1024 threads a strip, most without rows: max 125, 125, 41.5, 16.5 and
   // 68 f32; 112x15874 23.6 -> 6.8; 17920x128, whose second pass walked 280
   // partials in one workgroup, 49.3 -> 11.3.)
-  if (a.rows < 256) return cols_pass<E, E, KIND, 256>(a.src, a.ld, a.rows, a, nullptr, s);
+  if (a.rows < 256) return cols_pass<E, E, KIND, 256>(a.src, a.ld, a.rows, a, s);
   if (!a.workspace || (slots >= 200 * 16))
-    return cols_pass<E, E, KIND, 1024>(a.src, a.ld, a.rows, a, nullptr, s);
+    return cols_pass<E, E, KIND, 1024>(a.src, a.ld, a.rows, a, s);
   const ColsSplit sp = cols_split(a.rows, a.cols);
   const int run_log2 = sp.b_log2 - (8 - sp.sps_log2);  // rows a group: at most 2^12, 10 levels
 #define FRISK_BLOCKS(LV)                                                                             \
-  hipLaunchKernelGGL((reduce_cols_kernel<E, E, KIND, 256, LV>), dim3(sp.strips, sp.blocks), dim3(256), \
+  hipLaunchKernelGGL((reduce_cols_kernel<E, E, KIND, 256, LV, 0>), dim3(sp.strips, sp.blocks), dim3(256), \
                      0, s, a.src, a.ld, a.rows, a.cols, a.dst, a.dst_stride, a.clear, sp.sps_log2,    \
-                     run_log2, (float*)a.workspace)
+                     run_log2, 1, (float*)a.workspace)
   if (KIND != kReduceSum || run_log2 <= 8) FRISK_BLOCKS(6);
   else FRISK_BLOCKS(10);
 #undef FRISK_BLOCKS
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
-  return cols_pass<E, Elt::F32, KIND, 256>(a.workspace, a.cols, sp.blocks, a, nullptr, s);
+  return cols_pass<E, Elt::F32, KIND, 256>(a.workspace, a.cols, sp.blocks, a, s);
 }
 
 template <Elt E>
