@@ -585,9 +585,11 @@ int check_reduce(const frisk_reduce_desc* d, const char* fn) {
   return FRISK_OK;
 }
 
-// Bytes of workspace the two-pass axis-0 kernels take (0: single pass).
+// Bytes of workspace with which an axis-0 reduction takes two passes (0: one).
 int64_t reduce_workspace(const frisk_reduce_desc* d) {
-  if (d->axis != 0 || d->leaf_order_bits > 0 || d->rows < 256) return 0;
+  if (d->axis != 0 || d->leaf_order_bits > 0 ||
+      !frisk::plan::cols_two_pass(d->rows, d->cols, d->kind == FRISK_REDUCE_SUM, d->dtype == FRISK_F32))
+    return 0;
   const frisk::ColsSplit sp = frisk::cols_split(d->rows, d->cols);
   return sp.blocks * d->cols * (int64_t)sizeof(float);
 }

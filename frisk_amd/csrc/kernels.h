@@ -158,7 +158,7 @@ struct ReduceArgs {
   int order_bits;
   uint8_t order[32];
   // Axis 0 only: f32 scratch of cols_split(rows, cols).blocks * cols
-  // elements for the two-pass kernels, or null for the single pass.
+  // elements for two passes (plan::cols_two_pass), or null for one.
   void* workspace;
 };
 hipError_t tile_reduce(const ReduceArgs& a, hipStream_t s);

@@ -595,5 +595,25 @@ inline ColsPass cols_pass(int64_t rows, int64_t cols, bool sum, int threads) {
   return p;
 }
 
+// Whether a given workspace makes the launch take two passes: strips of rows
+// over the whole chip, then their f32 partials.  Under 256 rows, and from 3200
+// slots on where the strips of one pass do as well, one pass.  us, one pass
+// and two:
+//  * strips of 32 slots and more, f32 max 4096x32768 95.7 and 97.8, 8192x65536
+//    324 and 344, 20000x100000 1263 and 1334, bf16 sum 1024x65536 25.0 and 29.1;
+//  * strips of 8 or 16 slots that leave part of a CU round empty, f32 sum
+//    300x14000 7.7 and 10.8, 600x12801 15.9 and 12.5, 16384x13000 226 and 165,
+//    12000x20000 183 and 150, 65536x12800 679 and 558;
+//  * those that fill it, f32 max 2048x16384 22.9 and 24.7, 8192x16384 89.9 and
+//    87.7; f32 sums by 256 threads (32768x16384) 326 and 383.
+inline bool cols_two_pass(int64_t rows, int64_t cols, bool sum, bool f32) {
+  if (rows < 256) return false;
+  if ((cols + 3) / 4 < 3200) return true;
+  const ColsPass p = cols_pass(rows, cols, sum, 1024);
+  if (p.cvb_log2 > 4) return false;
+  if (!strips_fill(p.strips)) return rows >= 512;
+  return rows >= 8192 && !(f32 && sum && p.b_log2 > 8);
+}
+
 }  // namespace plan
 }  // namespace frisk

@@ -591,12 +591,10 @@ int ilog2(int64_t x) {
 }  // namespace
 
 ColsSplit cols_split(int64_t rows, int64_t cols) {
-  // One round of workgroups: pass 1 holds about 104 VGPRs, so 4 workgroups
-  // of 256 threads are resident per CU and 1024 fill the 256 CUs.  A sweep
-  // on 8192 x 16384 f32 (strips of 64 .. 1024 columns, row blocks of 8 ..
-  // 2^16 rows) peaked at exactly 1024 workgroups (4.0 TB/s; 2048 gave 3.7,
-  // 512 gave 2.6) with strips of 64 or 128 columns, whose 16 or 8 row groups
-  // keep each thread on a long run of rows.
+  // About 1024 workgroups of 256 threads: four fit a CU's registers.  (Swept
+  // on 8192 x 16384 f32 with the kernel before this one: 2048 and 512 were
+  // slower; strips of 64 or 128 columns, whose 16 or 8 row groups keep each
+  // thread on a long run of rows, the fastest.)
   ColsSplit sp;
   const int64_t slots = (cols + 3) / 4;
   sp.sps_log2 = ilog2(slots) < 5 ? ilog2(slots) : 5;
@@ -681,19 +679,11 @@ hipError_t reduce_typed(const ReduceArgs& a, hipStream_t s) {
 #undef FRISK_ROWS
     return hipGetLastError();
   }
-  const int64_t slots = (a.cols + 3) / 4;
-  // One pass of 1024-thread workgroups when strips of 16 slots (256 bytes of
-  // an f32 row) give at least 200 of them, or where there is no workspace;
-  // under 256 rows 256 threads.  Two passes otherwise, through f32 partials.
-  // One against two passes, us: f32 8192x16384 92.9 and 90.6, 4096x32768 96.4
-  // and 99.2, 2048x16384 25.3 and 27.3, 300x14000 8.3 and 12.1, bf16
-  // 1024x65536 26.8 and 31.5.  (Before, two passes from 256 rows on and below
-  // them 1024 threads a strip, most without rows: max 125, 125, 41.5, 16.5 and
-  // 68 f32; 112x15874 23.6 -> 6.8; 17920x128, whose second pass walked 280
-  // partials in one workgroup, 49.3 -> 11.3.)
+  // Two passes where plan::cols_two_pass asks for a workspace and the call has
+  // one; under 256 rows one pass of 256 threads a strip (f32 max of
+  // 112x15874 with 1024 threads, most of them without rows: 23.6 us, now 4.7).
   if (a.rows < 256) return cols_pass<E, E, KIND, 256>(a.src, a.ld, a.rows, a, s);
-  if (!a.workspace || (slots >= 200 * 16))
-    return cols_pass<E, E, KIND, 1024>(a.src, a.ld, a.rows, a, s);
+  if (!a.workspace) return cols_pass<E, E, KIND, 1024>(a.src, a.ld, a.rows, a, s);
   const ColsSplit sp = cols_split(a.rows, a.cols);
   const int run_log2 = sp.b_log2 - (8 - sp.sps_log2);  // rows a group: at most 2^12, 10 levels
 #define FRISK_BLOCKS(LV)                                                                             \

@@ -1,9 +1,12 @@
 """The launch geometry of axis-0 reductions (csrc/launch_plan.h), read by a
 host program."""
+import ctypes
 import os
 import subprocess
 
 import pytest
+
+from frisk_amd import runtime as rt
 
 CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "frisk_amd", "csrc")
 
@@ -54,3 +57,27 @@ def test_one_pass_covers_the_rows_on_live_threads(run):
         assert blocks < 1 << 12
         if blocks == 1 and threads == 1024:
             assert groups << b < 4 * rows or b == 3  # few idle row groups
+
+
+@pytest.mark.parametrize("dtype,kind", [(rt.F32, rt.REDUCE_SUM), (rt.F32, rt.REDUCE_MAX),
+                                        (rt.BF16, rt.REDUCE_SUM)])
+def test_workspace_query_asks_only_for_what_the_launch_reads(run, dtype, kind):
+    """The size is 0 exactly where frisk_reduce runs one pass, so no caller
+    allocates scratch nobody reads and no workspace is too short for it."""
+    plan = f"cols_two_pass(r, c, {str(kind == rt.REDUCE_SUM).lower()}, {str(dtype == rt.F32).lower()})"
+    lib = rt.load()
+    for (rows, cols), (two,) in zip(SHAPES, run([plan], SHAPES)):
+        d = rt.ReduceDesc(rows, cols, dtype, kind, 0, 1, 16, cols, 16, 1)
+        assert (lib.frisk_reduce_workspace_size(ctypes.byref(d)) > 0) == bool(two), (rows, cols)
+
+
+def test_one_pass_where_its_strips_fill_the_chip():
+    lib = rt.load()
+
+    def size(rows, cols, kind=rt.REDUCE_SUM, dtype=rt.F32):
+        d = rt.ReduceDesc(rows, cols, dtype, kind, 0, 1, 16, cols, 16, 1)
+        return lib.frisk_reduce_workspace_size(ctypes.byref(d))
+
+    assert size(1024, 65536) == 0 and size(4096, 32768, rt.REDUCE_MAX) == 0 and size(300, 14000) == 0
+    assert size(32768, 16384) == 0  # an f32 sum of long runs
+    assert size(16384, 13000) > 0 and size(600, 12801, dtype=rt.F16) > 0 and size(100000, 3) > 0
