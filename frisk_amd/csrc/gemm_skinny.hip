@@ -31,13 +31,13 @@
 //    slice order (deterministic) and converts.  Wider column tiles then cut
 //    the number of times X is streamed from L2 (every workgroup reads the
 //    X rows of its K range), and the slices restore the parallelism.
-//  * 8-bit types (M <= 64, never split: plan::skinny_plan).  Against 128x128
-//    tiles, which they ran on before, operands from HBM, us: fp8 32x8192x8192
-//    29.0 -> 17.2, 16x4096x4096 16.1 -> 8.1, 16x4096x14336 47.8 -> 14.5; int8
-//    16x14336x4096 16.6 -> 12.7, 64x4096x4096 16.9 -> 10.1.  What bounds them
-//    now is X, which every workgroup reads whole through L2 beside its W (the
-//    same with 8 or 16 waves per workgroup).
-//  * Roofline: HBM-bound; algorithmic bytes = M.K.2 + N.K.2 + M.N.2.
+//  * 8-bit types (M <= 64 where plan::skinny8_faster, never split).  Against
+//    128x128 tiles, operands from HBM, us: fp8 32x8192x8192 33.1 -> 21.0,
+//    16x4096x4096 17.9 -> 7.1, 16x4096x14336 52.5 -> 16.2; int8 16x14336x4096
+//    19.7 -> 16.8, 64x4096x4096 19.2 -> 11.7.  What bounds them now is X, which
+//    every workgroup reads whole through L2 beside its W (the same with 8 or
+//    16 waves per workgroup).
+//  * Roofline: HBM-bound; algorithmic bytes = (M.K + N.K).esize + M.N.2.
 
 #include <algorithm>
 

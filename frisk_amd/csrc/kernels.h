@@ -92,9 +92,9 @@ hipError_t gemm_128_split_layout(const GemmArgs& g, int slices, int64_t kb_slice
 hipError_t gemm_any(const GemmArgs& g, hipStream_t s, void* workspace, int64_t workspace_bytes);
 template <bool AM, bool BM>
 hipError_t gemm_any_layout(const GemmArgs& g, const plan::SplitPlan& p, void* ws, hipStream_t s);
-// Small-M kernel (plan::skinny_supported: M <= kSkinnyMaxM, bf16/f16,
-// trans_a == 0, trans_b == 1, 16 B aligned K-contiguous rows);
-// memory-bound regime.
+// Small-M kernel (plan::skinny_supported: bf16/f16 up to kSkinnyMaxM rows, the
+// 8-bit types up to kSkinnyMaxM8; trans_a == 0, trans_b == 1, 16 B aligned
+// K-contiguous rows); memory-bound regime.
 using plan::kSkinnyMaxM;
 inline bool gemm_skinny_supported(const GemmArgs& g) { return plan::skinny_supported(shape_of(g)); }
 inline SkinnyPlan gemm_skinny_plan(const GemmArgs& g, int cus, bool split) {

@@ -44,8 +44,7 @@ constexpr int64_t kSkinnyMaxM = FRISK_SKINNY_MAX_M;
 // more (up to its limit) run split on 128x128 tiles, which share each X
 // tile across the workgroup's waves through LDS.
 constexpr int64_t kSkinnySplitMaxM = 64;
-// 8-bit inputs: past 64 rows the 128x128 tiles are as fast or faster (fp8
-// 128x8192x8192 30.3 us against 39.0).
+// 8-bit inputs: the most rows on the small-M kernel, where skinny8_faster.
 constexpr int64_t kSkinnyMaxM8 = 64;
 // Split-K arrival words per tile of the in-launch slice sum (gemm_common.h
 // splitk_tree) and the most slices summed that way on 128x128 tiles.
@@ -272,13 +271,35 @@ inline int stage_bytes_128(const GemmShape& g, int cus) {
 }
 
 // ---------------------------------------------------------------------------
-// Small-M kernel (M <= kSkinnyMaxM, bf16/f16, A [M, K], B [N, K]): TM x TN
-// 16x16 atoms per workgroup (4 waves), `slices` K slices of
+// Small-M kernel (M <= kSkinnyMaxM, A [M, K], B [N, K]): TM x TN 16x16 atoms per workgroup (4 waves), `slices` K slices of
 // steps_per_slice 64-byte k-steps, and the f32 workspace the slices'
 // partial tiles need (0 without split-K).
 // ---------------------------------------------------------------------------
+// 8-bit inputs: the shapes on which the small-M kernel beats the tiles they
+// would run on, whose time hardly grows up to 128 rows: 128x128, and 256x256
+// from 32768 columns on.  Measured over N 16 .. 100000, K 16 .. 16384, W from
+// HBM, small-M / tile time at M 16, 32, 64 (fp8; int8 within 0.1 of it):
+//   N  4096  K 4096   0.39 0.49 0.59     N  8192  K  4096  0.54 0.67 0.90
+//   N  8192  K  512   0.71 0.76 1.05     N  8192  K   128  0.82 0.88 1.15
+//   N 14336  K 4096   0.85 0.96 1.23     N 14336  K   512  0.91 1.07 1.36
+//   N 20480  K 4096   1.19 1.38 1.96     N 28672  K  4096  1.03 1.16 1.64
+//   N 32768  K 4096   0.65 0.73 1.04     N 57344  K  2048  0.98 1.05 1.75
+// So: one round of 32-column tiles, past 32 rows only where the 128x128 tiles
+// are few (N 4096) or K is not short; one round of 64-column tiles up to 16
+// rows, or 32 with a long K; two rounds of them only nearly whole, for up to
+// 8 rows and a long K; against 256x256 tiles up to 16 rows, or 32 while those
+// are one round or K is short (M 32, N 50000, K 4096: 1.10).
+inline bool skinny8_faster(const GemmShape& g) {
+  if (g.n <= 4096) return true;
+  if (g.n <= 8192) return g.m <= 32 || g.k >= 512;
+  if (g.n <= 16384) return g.m <= 16 || (g.m <= 32 && g.k >= 1024);
+  if (g.n < 32768) return g.m <= 8 && g.n >= 28672 && g.k >= 4096;
+  return g.m <= 16 || (g.m <= 32 && (g.n <= 49152 || g.k <= 1024));
+}
+
 inline bool skinny_supported(const GemmShape& g) {
-  if (g.in == kE4M3 || g.in == kI8) return g.m <= kSkinnyMaxM8 && !g.trans_a && g.trans_b;
+  if (g.in == kE4M3 || g.in == kI8)
+    return g.m <= kSkinnyMaxM8 && !g.trans_a && g.trans_b && skinny8_faster(g);
   const bool type_ok = (g.in == kBF16 && (g.out == kBF16 || g.out == kF32)) ||
                        (g.in == kF16 && (g.out == kF16 || g.out == kF32));
   return type_ok && g.m <= kSkinnyMaxM && !g.trans_a && g.trans_b;
@@ -300,10 +321,10 @@ inline SkinnyPlan skinny_plan(const GemmShape& g, int cus, bool split) {
   p.workspace_bytes = 0;
   if (g.in == kE4M3 || g.in == kI8) {
     // The narrowest columns whose tiles fit the CUs in one round, else the
-    // widest, unsplit (us, 16-, 32-, 64-column tiles, and two slices of the
-    // best: fp8 32x8192x8192 24.1, 17.2, 21.3, 18.4; 16x4096x4096 8.0, 8.1,
-    // 12.1, 12.3; 64x8192x8192 31, 26.1, 26.4, 26.4; int8 16x14336x4096 17.5,
-    // 13.7, 12.7, 16.8).
+    // widest, unsplit (us, operands in the last-level cache, 16-, 32-,
+    // 64-column tiles, and two slices of the best: fp8 32x8192x8192 24.1,
+    // 17.2, 21.3, 18.4; 16x4096x4096 8.0, 8.1, 12.1, 12.3; 64x8192x8192 31,
+    // 26.1, 26.4, 26.4; int8 16x14336x4096 17.5, 13.7, 12.7, 16.8).
     const int64_t rows = (g.m + 16 * p.tm - 1) / (16 * p.tm);
     p.tn = 1;
     while (p.tn < 4 && (g.n + 16 * p.tn - 1) / (16 * p.tn) * rows > (cus > 0 ? cus : 256)) p.tn *= 2;

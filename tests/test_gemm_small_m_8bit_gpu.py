@@ -15,9 +15,10 @@ pytestmark = pytest.mark.gpu
 FP8 = torch.float8_e4m3fn
 # K inside one 16-byte piece and one 64-byte step, whole batches and a tail;
 # N partial in the last tile, one round of 16-column tiles (4096), wider
-# columns (8192: 32, 24584: 64); M at each tile height and one past it.
+# columns (8192: 32, 16328: 64); M at each tile height and one past it.  Past
+# 32 rows the wide ones (24584, 8200) run on 128x128 tiles.
 SHAPES = [(1, 16, 16), (5, 40, 48), (16, 4096, 1040), (17, 72, 2064), (32, 8192, 256), (33, 24584, 80),
-          (64, 4096, 192), (64, 8200, 64)]
+          (64, 4096, 192), (64, 8200, 64), (16, 16328, 80), (32, 8200, 1040), (64, 8184, 1040)]
 
 
 @pytest.mark.parametrize("in_dt,out_dt", [(FP8, torch.bfloat16), (FP8, torch.float16),
@@ -37,7 +38,8 @@ def test_small_m_8bit(in_dt, out_dt):
         c.t.zero_()
         out = c.t[:, :n]
         kw = dict(trans_b=True, scale_a=sa, scale_b=sb)
-        assert rt.gemm_plan(a, b, out, trans_b=True)["kernel"] == "gemm_skinny"
+        want = "gemm_128" if m > 32 and n >= 8200 else "gemm_skinny"
+        assert rt.gemm_plan(a, b, out, trans_b=True)["kernel"] == want
         ref = G.gemm_int(decode(a), decode(b), trans_b=True) if in_dt == torch.int8 else \
             G.gemm_fp64(decode(a), decode(b), trans_b=True) * (sa * sb)
         for times in (1, 2):  # C = A.B, then C += A.B
