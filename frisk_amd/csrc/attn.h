@@ -618,19 +618,16 @@ static hipError_t launch_attn_nw(const AttnArgs& a, hipStream_t stream) {
   return hipGetLastError();
 }
 
-// Workgroup shape per launch: a.waves when the request names one, else
-// plan::attn_waves (launch_plan.h, which holds the measurements behind the
-// rule).  Head_dim 64 and below run 4-wave workgroups only.  Every query's
-// arithmetic is the same in both shapes (same key blocks in the same order;
-// a masked block with no hidden key computes what an unmasked one does), so
-// the choice never changes a result bit.
+// Workgroup shape per launch (plan::attn_launch, which holds the measurements
+// behind the rule).  Head_dim 64 and below run 4-wave workgroups only.  Every
+// query's arithmetic is the same in both shapes (same key blocks in the same
+// order; a masked block with no hidden key computes what an unmasked one
+// does), so the choice never changes a result bit.
 template <Elt T, Elt OUT, int D, bool CAUSAL, bool KT>
-static hipError_t launch_attn_kt(const AttnArgs& a, hipStream_t stream) {
+static hipError_t launch_attn_kt(const AttnArgs& a, int waves, hipStream_t stream) {
   if constexpr (D <= 64) {
     return launch_attn_nw<T, OUT, D, 4, CAUSAL, KT>(a, stream);
   } else {
-    const int waves = a.waves ? a.waves
-                              : plan::attn_waves(a.batch * a.heads, a.seq_q, D, CAUSAL, device_cus());
     return waves == 4 ? launch_attn_nw<T, OUT, D, 4, CAUSAL, KT>(a, stream)
                       : launch_attn_nw<T, OUT, D, 8, CAUSAL, KT>(a, stream);
   }
@@ -640,16 +637,16 @@ static hipError_t launch_attn_kt(const AttnArgs& a, hipStream_t stream) {
 template <Elt T, Elt OUT, int D, bool CAUSAL, bool KT>
 static hipError_t launch_fewq(const AttnArgs& a, hipStream_t stream);
 
-// K stored [.., seq, head_dim] or [.., head_dim, seq] (a.k_dmajor).  Up to
-// kFewQ queries run one query tile whose waves divide the keys, whatever
-// `waves` names.
+// K stored [.., seq, head_dim] or [.., head_dim, seq] (a.k_dmajor).
 template <Elt T, Elt OUT, int D, bool CAUSAL>
 static hipError_t launch_attn(const AttnArgs& a, hipStream_t stream) {
-  if (a.seq_q <= plan::kFewQ)
+  const plan::AttnLaunch L =
+      plan::attn_launch(a.batch * a.heads, a.seq_q, a.seq_k, D, CAUSAL, device_cus(), a.waves);
+  if (L.few)
     return a.k_dmajor ? launch_fewq<T, OUT, D, CAUSAL, true>(a, stream)
                       : launch_fewq<T, OUT, D, CAUSAL, false>(a, stream);
-  return a.k_dmajor ? launch_attn_kt<T, OUT, D, CAUSAL, true>(a, stream)
-                    : launch_attn_kt<T, OUT, D, CAUSAL, false>(a, stream);
+  return a.k_dmajor ? launch_attn_kt<T, OUT, D, CAUSAL, true>(a, L.waves, stream)
+                    : launch_attn_kt<T, OUT, D, CAUSAL, false>(a, L.waves, stream);
 }
 
 // Every (input dtype, output dtype, mask) variant of one head_dim.

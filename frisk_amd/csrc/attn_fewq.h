@@ -1,5 +1,5 @@
-// Attention forward for few queries (seq_q <= 32: decode steps) on gfx950:
-// one workgroup per (batch, head) and key split, whose waves share one tile
+// Attention forward for few queries (seq_q <= 32: decode steps) and enough keys
+// (plan::attn_few) on gfx950: one workgroup per (batch, head) and key split, whose waves share one tile
 // of 32 queries and divide the keys.
 //
 // attn.h gives every wave queries of its own and walks the keys together, one
@@ -28,7 +28,7 @@ namespace fewq {
 constexpr int kMaxQ = plan::kFewQ;
 
 // Waves per workgroup: K and V tiles of all waves take 96 to 128 KiB of LDS.
-template <int D> constexpr int kWaves = D == 128 ? 4 : D == 64 ? 8 : 16;
+template <int D> constexpr int kWaves = plan::few_waves(D);
 
 template <int D> constexpr int lds_bytes() {
   const int tiles = kWaves<D> * AttnGeom<D>::kBuf;

@@ -116,7 +116,7 @@ struct AttnArgs {
   const void* k;
   int64_t k_sb, k_sh, k_ss;  // k_ss: between keys, or with k_dmajor between head_dim rows
   int k_dmajor;              // K stored [batch, heads, head_dim, seq]
-  int waves = 0;             // waves per workgroup (4 or 8); 0: plan::attn_waves
+  int waves = 0;             // waves per workgroup (4 or 8) of attn.h; 0: plan::attn_waves
   const void* v;
   int64_t v_sb, v_sh, v_ss;
   void* o;

@@ -525,21 +525,50 @@ inline int attn_waves(int64_t batch_heads, int64_t seq_q, int64_t head_dim, bool
   return t4 < t8 ? 4 : 8;
 }
 
-// Few queries (decode steps): up to kFewQ, one query tile, run the kernel
-// whose waves divide the keys (attn_fewq.h) in `attn_splits` key splits per
-// head, combined by a second launch from the f32 rows of attn_workspace.
-// A workgroup's round of key blocks (64 keys per wave) takes about 2.2 us of
-// a CU, all of K and V at least their bytes at 6 TB/s, a split about 5 us of
-// second launch and scratch and 0.15 us to read each split's rows.  Measured, us, 1 -> the chosen splits -> twice
-// that: b1 h32 s4096 d128 31.4 -> 16.7 (4) -> 18.4; b1 h1 s32768 d128 217 ->
-// 22.3 (32); b4 h32 s4096 d128 50.6 (1) -> 51.1; b5 h16 s2432 d64 11.9 (1) ->
-// 13.0.  (The kernel before, whose waves did not divide the keys: 81 us at b4
-// h32 s4096, 29.3 at b5 h16 s2432 d64, 48.2 at b64 h4 s5231 d16, now 16.6.)
+// Few queries (decode steps): up to kFewQ, one query tile, and enough blocks of
+// 64 keys run the kernel whose waves divide the keys (attn_fewq.h).  Its
+// workgroup holds a CU (96 to 128 KiB of LDS) with few_waves waves, of which
+// seq_k / 64 have keys, where several of attn.h's share one; it pays from two
+// to four key blocks on while the heads are one round of workgroups, later in
+// several rounds.  Measured, attn_fewq / attn.h time, one query, at 32, 256,
+// 1024 and 8192 heads:
+//   d 16   128 keys 1.16 1.16 2.01 2.75    256 0.92 0.99 1.51 1.80   768 0.61 0.66 0.89 0.97
+//   d 64   128 keys 1.04 1.07 1.49 1.76    256 0.83 0.96 1.17 1.43   768 0.56 0.74 0.90  -
+//   d 128   64 keys 1.15 1.02 1.45 1.74    128 0.95 0.98 1.28 1.39   512 0.67 0.86 0.92  -
 constexpr int64_t kFewQ = 32;
+constexpr int few_waves(int64_t head_dim) { return head_dim == 128 ? 4 : head_dim == 64 ? 8 : 16; }
 
-inline int attn_splits(int64_t batch_heads, int64_t seq_q, int64_t seq_k, int64_t head_dim, int cus) {
+inline bool attn_few(int64_t batch_heads, int64_t seq_q, int64_t seq_k, int64_t head_dim, int cus) {
   const int64_t nkb = (seq_k + 63) / 64;
-  const int64_t waves = head_dim == 128 ? 4 : head_dim == 64 ? 8 : 16;
+  if (seq_q > kFewQ || batch_heads * 64 * few_waves(head_dim) > UINT32_MAX) return false;  // (threads of a grid)
+  if (batch_heads <= cus) return nkb >= (head_dim == 128 ? 2 : head_dim == 64 ? 3 : 4);
+  return nkb >= (head_dim == 128 ? 7 : 12);
+}
+
+// The kernel and waves per workgroup of a call; `waves` (4, 8 or 0) chooses
+// among attn.h's workgroups.
+struct AttnLaunch {
+  bool few;
+  int waves;
+};
+inline AttnLaunch attn_launch(int64_t batch_heads, int64_t seq_q, int64_t seq_k, int64_t head_dim,
+                              bool causal, int cus, int waves) {
+  if (attn_few(batch_heads, seq_q, seq_k, head_dim, cus)) return AttnLaunch{true, few_waves(head_dim)};
+  return AttnLaunch{false, waves ? waves : attn_waves(batch_heads, seq_q, head_dim, causal, cus)};
+}
+
+// The few-query kernel runs `attn_splits` key splits per head, combined by a
+// second launch from the f32 rows of attn_workspace.  A workgroup's round of
+// key blocks (64 keys per wave) takes about 2.2 us of a CU, all of K and V at
+// least their bytes at 6 TB/s, a split about 5 us of second launch and scratch
+// and 0.15 us to read each split's rows.  Measured, us, 1 -> the chosen splits
+// -> twice that: b1 h32 s4096 d128 31.4 -> 16.7 (4) -> 18.4; b1 h1 s32768 d128
+// 217 -> 22.3 (32); b4 h32 s4096 d128 50.6 (1) -> 51.1; b5 h16 s2432 d64 11.9
+// (1) -> 13.0.  (The kernel before, whose waves did not divide the keys: 81 us
+// at b4 h32 s4096, 29.3 at b5 h16 s2432 d64, 48.2 at b64 h4 s5231 d16, now
+// 16.6.)
+inline int attn_splits(int64_t batch_heads, int64_t seq_q, int64_t seq_k, int64_t head_dim, int cus) {
+  const int64_t nkb = (seq_k + 63) / 64, waves = few_waves(head_dim);
   // (Up to 12 key blocks no split gains: callers ask for a workspace past
   // that only.)
   if (nkb <= 12) return 1;
@@ -559,7 +588,7 @@ inline int attn_splits(int64_t batch_heads, int64_t seq_q, int64_t seq_k, int64_
 }
 inline int64_t attn_workspace(int64_t batch_heads, int64_t seq_q, int64_t seq_k, int64_t head_dim,
                               int cus) {
-  if (seq_q > kFewQ) return 0;
+  if (!attn_few(batch_heads, seq_q, seq_k, head_dim, cus)) return 0;
   const int64_t s = attn_splits(batch_heads, seq_q, seq_k, head_dim, cus);
   return s > 1 ? batch_heads * s * seq_q * (head_dim + 2) * 4 : 0;
 }

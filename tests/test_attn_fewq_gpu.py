@@ -19,8 +19,11 @@ LSE_TOL = {torch.bfloat16: 4e-3, torch.float16: 1e-3}
 # (batch, heads, seq_q, seq_k): fewer blocks of 64 keys than waves, one past
 # and one short of a block, a whole round of blocks, more queries than keys,
 # the most queries of the kernel, and lengths that split over the workspace.
+# (The shortest run the query-tiled kernel, by head_dim: plan::attn_few; the
+# fewest keys of this one, and more heads than one round of its workgroups.)
 CASES = [(1, 1, 1, 1), (1, 2, 1, 63), (2, 1, 3, 65), (1, 3, 1, 1024), (1, 2, 32, 33), (1, 1, 32, 7),
-         (2, 2, 17, 300), (1, 2, 1, 4097), (1, 1, 5, 9000)]
+         (2, 2, 17, 300), (1, 2, 1, 4097), (1, 1, 5, 9000), (1, 2, 32, 129), (2, 1, 32, 193), (1, 1, 1, 193),
+         (3, 100, 2, 706)]
 
 
 def call(q, k, v, o, lse, causal, ws, **kw):
