@@ -316,12 +316,15 @@ GemmLaunchContract cdna4GemmLaunch(int64_t m, int64_t n, int64_t k, Type in, Typ
   return c;
 }
 
-int64_t cdna4AttentionWaves(int64_t batchHeads, int64_t seqQ, int64_t headDim, bool causal,
-                            int64_t cus) {
-  if (batchHeads <= 0 || seqQ <= 0) throw InvalidArgument("launch contract: sizes must be positive");
+AttentionLaunchContract cdna4AttentionLaunch(int64_t batchHeads, int64_t seqQ, int64_t seqK,
+                                             int64_t headDim, bool causal, int64_t cus) {
+  if (batchHeads <= 0 || seqQ <= 0 || seqK <= 0)
+    throw InvalidArgument("launch contract: sizes must be positive");
   if (headDim != 16 && headDim != 32 && headDim != 64 && headDim != 128)
     throw InvalidArgument("launch contract: the attention kernel takes head_dim 16, 32, 64 or 128");
-  return frisk::plan::attn_waves(batchHeads, seqQ, headDim, causal, (int)cus);
+  const frisk::plan::AttnLaunch L =
+      frisk::plan::attn_launch(batchHeads, seqQ, seqK, headDim, causal, (int)cus, 0);
+  return AttentionLaunchContract{L.few ? "attn_fewq" : "attn_fwd", L.waves};
 }
 
 }  // namespace fir

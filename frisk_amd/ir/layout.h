@@ -127,7 +127,14 @@ struct GemmLaunchContract {
 // meet the MFMA kernels' alignment and reach conditions.
 GemmLaunchContract cdna4GemmLaunch(int64_t m, int64_t n, int64_t k, Type in, Type out, bool transA,
                                    bool transB, int64_t cus, bool workspace, bool matrixCores);
-int64_t cdna4AttentionWaves(int64_t batchHeads, int64_t seqQ, int64_t headDim, bool causal,
-                            int64_t cus);
+// The attention kernel of a program and its waves per workgroup: "attn_fwd"
+// (32 queries per wave; what frisk_attn_desc.waves names) or "attn_fewq" (one
+// tile of up to 32 queries, the waves divide the keys).
+struct AttentionLaunchContract {
+  std::string kernel;
+  int64_t waves = 0;
+};
+AttentionLaunchContract cdna4AttentionLaunch(int64_t batchHeads, int64_t seqQ, int64_t seqK,
+                                             int64_t headDim, bool causal, int64_t cus);
 
 }  // namespace fir

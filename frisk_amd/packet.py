@@ -315,8 +315,9 @@ def execute_packet(packet, tensors, *, stream=None, require_layout_match=False,
     else:
         q, k, v, o = (tensors[plan[n]] for n in ("q", "k", "v", "o"))
         view = lambda t: t.view(1, 1, *t.shape)
-        plan["waves"] = _ir().frisk.attention_launch_plan(1, q.shape[0], q.shape[1], False,
-                                                          _device_cus())["waves"]
+        L = _ir().frisk.attention_launch_plan(1, q.shape[0], q.shape[1], False, _device_cus(),
+                                              seq_k=v.shape[0])
+        plan["waves"] = L["waves"]
         rt.attn_fwd(view(q), view(k), view(v), view(o), causal=False, sm_scale=plan["scale"],
-                    stream=stream, waves=plan["waves"])
+                    stream=stream, waves=rt.requested_waves(L))
     return plan

@@ -359,9 +359,15 @@ def attn_desc(q, k, v, o, *, causal=False, sm_scale=None, lse=None,
                     int(bool(k_transposed)), int(waves))
 
 
-# frisk_attn_fwd_ws splits the keys of calls with at most FEW_QUERIES queries
-# and more than FEW_KEYS keys.
+# frisk_attn_fwd_ws splits the keys only of calls with at most FEW_QUERIES
+# queries and more than FEW_KEYS keys.
 FEW_QUERIES, FEW_KEYS = 32, 768
+
+
+def requested_waves(contract: dict) -> int:
+    """AttnDesc.waves of an attention launch contract: the waves of the kernel
+    that gives every wave its own queries; the few-query kernel takes none."""
+    return contract["waves"] if contract["kernel"] == "attn_fwd" else 0
 
 
 def attn_fwd(q, k, v, o, *, causal=False, sm_scale=None, lse=None, stream=None,

@@ -216,7 +216,11 @@ typedef struct frisk_attn_desc {
   int32_t k_transposed; /* 0: K [b, h, seq_k, head_dim]; 1: K [b, h, head_dim, seq_k] */
   /* Waves per workgroup (32 queries each): 0, the library chooses (the
    * launch contract layout inference gives an attention program); 4 or 8
-   * (8 needs head_dim 128).  The result bits do not depend on it. */
+   * (8 needs head_dim 128).  A call that the few-query kernel takes (up to
+   * 32 queries and more than 64 to 704 keys, by head_dim and the number of
+   * heads; "attn_fewq" in the launch contract), whose 4, 8 or 16 waves divide
+   * the keys, is checked for it and runs the same with any.  The result bits
+   * do not depend on it. */
   int32_t waves;
 } frisk_attn_desc;
 

@@ -1,8 +1,13 @@
-"""Which attention kernel a call gets (csrc/launch_plan.h)."""
+"""Which attention kernel a call gets (csrc/launch_plan.h): the target's launch
+contract reports what the library launches."""
+import ctypes
 import os
 import subprocess
 
 import pytest
+
+import frisk_amd as F
+from frisk_amd import runtime as rt
 
 CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "frisk_amd", "csrc")
 
@@ -35,3 +40,35 @@ def test_few_queries_need_enough_keys_for_their_heads(few, d, waves):
     # A grid of workgroups holds fewer than 2^32 threads.
     most = (1 << 32) // (64 * waves)
     assert few([(most - 1, 1, 4096, d), (most, 1, 4096, d)]) == [True, False]
+
+
+def contract(bh, sq, sk, d):
+    L = F.frisk.attention_launch_plan(bh, sq, d, seq_k=sk)
+    return L["kernel"], L["waves"]
+
+
+@pytest.mark.parametrize("d,waves", [(16, 16), (32, 16), (64, 8), (128, 4)])
+def test_launch_contract_reports_the_few_query_kernel(few, d, waves):
+    calls = [(bh, sq, sk, d) for bh in (1, 256, 8192) for sq in (1, 32, 33) for sk in (64, 200, 1000)]
+    for c, is_few in zip(calls, few(calls)):
+        kernel, got = contract(*c)
+        assert kernel == ("attn_fewq" if is_few else "attn_fwd")
+        assert got == waves if is_few else got in (4, 8)
+    # The keys default to the queries: a square problem of few queries has few keys.
+    assert F.frisk.attention_launch_plan(64, 32, d)["kernel"] == "attn_fwd"
+
+
+def test_waves_requested_are_those_of_the_query_tiled_kernel():
+    assert rt.requested_waves(F.frisk.attention_launch_plan(128, 4096, 128)) == 8
+    assert rt.requested_waves(F.frisk.attention_launch_plan(8, 4, 16, seq_k=4096)) == 0
+
+
+@pytest.mark.parametrize("bh,sq,sk,d", [(2, 1, 4096, 128), (256, 1, 832, 64), (2, 32, 9000, 16),
+                                        (2, 33, 9000, 128), (2, 1, 768, 128), (8192, 1, 512, 64)])
+def test_scratch_only_for_the_few_query_kernel(bh, sq, sk, d):
+    a = rt.AttnDesc(bh, 1, sq, sk, d, rt.BF16, 0, 1.0, 0, sq * d, sq * d, d, 0, sk * d, sk * d, d,
+                    0, sk * d, sk * d, d, 0, sq * d, sq * d, d, None, rt.BF16, 0, 0)
+    need = rt.load().frisk_attn_workspace_size(ctypes.byref(a))
+    assert need >= 0, rt.load().frisk_last_error()
+    if contract(bh, sq, sk, d)[0] != "attn_fewq" or sk <= rt.FEW_KEYS:
+        assert need == 0
