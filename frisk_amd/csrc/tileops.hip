@@ -439,13 +439,16 @@ constexpr int kSlots = 4;  // 8-element slots per thread
 // Slot s of row r holds columns [8 s, 8 s + 8).  A thread works on kSlots of
 // them, its loads first and its stores after, so that kSlots loads are in
 // flight.  WIDE: thread t of block x takes slots (x kSlots + u) 256 + t, u <
-// kSlots, of rows y, y + gridDim.y, ...  Rows of at most 128 slots share a
-// workgroup instead, 2^tpr_log2 threads each: with a workgroup per row a
+// kSlots, of rows y, y + gridDim.y, ...  Short rows share a workgroup instead,
+// 2^tpr_log2 threads each, spt slots a thread: with a workgroup per row a
 // [30000, 136] copy kept 17 of 256 threads busy (23.3 -> 6.7 us).
 // load(u, r, c) and store(u, r, c) are called for every slot inside.
+// (The tails of conversions are loops neither unrolled nor vectorised: those
+// took registers, 93 against 68 for fp8 -> bf16, and waves: 16384x8192 91 -> 75
+// us.)
 template <bool WIDE, typename Load, typename Store>
-__device__ __forceinline__ void each_slot(int64_t rows, int64_t cols, int tpr_log2, Load load,
-                                          Store store) {
+__device__ __forceinline__ void each_slot(int64_t rows, int64_t cols, int tpr_log2, int spt,
+                                          Load load, Store store) {
   using namespace tile;
   if constexpr (WIDE) {
     for (int64_t r = blockIdx.y; r < rows; r += gridDim.y) {
@@ -465,14 +468,15 @@ __device__ __forceinline__ void each_slot(int64_t rows, int64_t cols, int tpr_lo
     const int64_t c = (int64_t)(threadIdx.x & ((1 << tpr_log2) - 1)) * 8;
     if (c >= cols) return;
     const int sub = threadIdx.x >> tpr_log2;
-    for (int64_t r0 = (int64_t)blockIdx.x * rpp * kSlots; r0 < rows;
-         r0 += (int64_t)gridDim.x * rpp * kSlots) {
+    for (int64_t r0 = (int64_t)blockIdx.x * rpp * spt; r0 < rows;
+         r0 += (int64_t)gridDim.x * rpp * spt) {
+      const int64_t end = min(rows, r0 + (int64_t)rpp * spt);
 #pragma unroll
       for (int u = 0; u < kSlots; ++u)
-        if (r0 + u * rpp + sub < rows) load(u, r0 + u * rpp + sub, c);
+        if (r0 + u * rpp + sub < end) load(u, r0 + u * rpp + sub, c);
 #pragma unroll
       for (int u = 0; u < kSlots; ++u)
-        if (r0 + u * rpp + sub < rows) store(u, r0 + u * rpp + sub, c);
+        if (r0 + u * rpp + sub < end) store(u, r0 + u * rpp + sub, c);
     }
   }
 }
@@ -487,10 +491,12 @@ template <typename Raw> __device__ __forceinline__ void store_any(void* p, const
   typedef Raw Any __attribute__((aligned(1)));
   *(Any*)p = v;
 }
-// A copy's output: past the caches when a lane's eight elements are at most 16
-// bytes, whole lines per wave (16384x8192 bf16 -> f16 96.1 -> 92.9 us,
-// 8192x2048 f32 -> bf16 18.2 -> 15.1; as two halves of 32 bytes f32 188 ->
-// 326).
+// A converted output: past the caches when a lane's eight elements are at most
+// 16 bytes, whole lines per wave (us: 16384x8192 bf16 -> f16 96.1 -> 92.9, f32 ->
+// bf16 144 -> 140; as two halves of 32 bytes f32 188 -> 326).  Copies of one
+// type are faster through them (bf16 200000x256 46 -> 36, 2000x16384 26.5 ->
+// 24.9, fp8 16384x8192 46 -> 43), short rows of bytes apart (fp8 200000x300 47
+// through them, 37).
 template <typename Raw> __device__ __forceinline__ void store_stream(void* p, const Raw& v) {
   typedef Raw Any __attribute__((aligned(1)));
   if constexpr (sizeof(Raw) <= 16) __builtin_nontemporal_store(v, (Any*)p);
@@ -501,14 +507,14 @@ template <typename Raw> __device__ __forceinline__ void store_stream(void* p, co
 template <Elt S, Elt D, bool WIDE>
 __global__ __launch_bounds__(tile::kThreads) void copy_convert_kernel(
     const void* __restrict__ src, int64_t ld_src, void* __restrict__ dst, int64_t ld_dst,
-    int64_t rows, int64_t cols, int tpr_log2) {
+    int64_t rows, int64_t cols, int tpr_log2, int spt) {
   using namespace tile;
   constexpr int kSe = EltInfo<S>::bytes, kDe = EltInfo<D>::bytes;
   using SRaw = typename Raw8<kSe>::T;
   using DRaw = typename Raw8<kDe>::T;
   SRaw in[kSlots];
   each_slot<WIDE>(
-      rows, cols, tpr_log2,
+      rows, cols, tpr_log2, spt,
       [&](int u, int64_t r, int64_t c) {
         if (c + 8 <= cols) in[u] = load_any<SRaw>((const char*)src + (r * ld_src + c) * kSe);
       },
@@ -521,6 +527,7 @@ __global__ __launch_bounds__(tile::kThreads) void copy_convert_kernel(
           convert8<D>(x, &out);
           store_stream<DRaw>((char*)dst + (r * ld_dst + c) * kDe, out);
         } else {
+#pragma clang loop vectorize(disable) unroll(disable)
           for (; c < cols; ++c) put<D>(dst, r * ld_dst + c, load_as_f32<S>(src, r * ld_src + c));
         }
       });
@@ -537,7 +544,7 @@ using WordOf = typename std::conditional<
 template <int BYTES, bool WIDE>
 __global__ __launch_bounds__(tile::kThreads) void copy_raw_kernel(
     const void* __restrict__ src, int64_t ld_src, void* __restrict__ dst, int64_t ld_dst,
-    int64_t rows, int64_t cols, int tpr_log2) {
+    int64_t rows, int64_t cols, int tpr_log2, int spt) {
   using namespace tile;
   using Raw = typename Raw8<BYTES>::T;
   using Word = WordOf<BYTES>;
@@ -545,14 +552,21 @@ __global__ __launch_bounds__(tile::kThreads) void copy_raw_kernel(
   Word* dp = (Word*)dst;
   Raw in[kSlots];
   each_slot<WIDE>(
-      rows, cols, tpr_log2,
+      rows, cols, tpr_log2, spt,
       [&](int u, int64_t r, int64_t c) {
         if (c + 8 <= cols) in[u] = load_any<Raw>(sp + r * ld_src + c);
       },
       [&](int u, int64_t r, int64_t c) {
-        if (c + 8 <= cols) store_stream<Raw>(dp + r * ld_dst + c, in[u]);
-        else
+        if (c + 8 <= cols) {
+          if constexpr (BYTES == 1 && !WIDE) store_stream<Raw>(dp + r * ld_dst + c, in[u]);
+          else store_any<Raw>(dp + r * ld_dst + c, in[u]);
+        } else if constexpr (BYTES == 8) {  // (as a loop 100 registers, so 75)
+#pragma unroll
+          for (int i = 0; i < 8; ++i)
+            if (c + i < cols) dp[r * ld_dst + c + i] = sp[r * ld_src + c + i];
+        } else {
           for (; c < cols; ++c) dp[r * ld_dst + c] = sp[r * ld_src + c];
+        }
       });
 }
 
@@ -560,7 +574,7 @@ __global__ __launch_bounds__(tile::kThreads) void copy_raw_kernel(
 template <int BYTES, bool WIDE>
 __global__ __launch_bounds__(tile::kThreads) void fill_kernel(void* __restrict__ dst, int64_t ld,
                                                               int64_t rows, int64_t cols,
-                                                              uint64_t bits, int tpr_log2) {
+                                                              uint64_t bits, int tpr_log2, int spt) {
   using namespace tile;
   using Raw = typename Raw8<BYTES>::T;
   using Word = WordOf<BYTES>;
@@ -570,7 +584,7 @@ __global__ __launch_bounds__(tile::kThreads) void fill_kernel(void* __restrict__
 #pragma unroll
   for (int i = 0; i < 8; ++i) pw[i] = (Word)bits;
   each_slot<WIDE>(
-      rows, cols, tpr_log2, [](int, int64_t, int64_t) {},
+      rows, cols, tpr_log2, spt, [](int, int64_t, int64_t) {},
       [&](int, int64_t r, int64_t c) {
         if (c + 8 <= cols) store_any<Raw>(dp + r * ld + c, pat);
         else
@@ -708,30 +722,38 @@ hipError_t reduce_kind(const ReduceArgs& a, hipStream_t s) {
   }
 }
 
-// Grid and threads per row of each_slot.
+// Grid, threads per row and slots per thread of each_slot.
 struct SlotGrid {
   dim3 grid;
-  int tpr_log2;
+  int tpr_log2, spt;
 };
-SlotGrid slot_grid(int64_t rows, int64_t cols) {
+// Rows of up to most_slots slots share workgroups, and a thread takes as many
+// slots as leave fill_blocks workgroups: two per CU for conversions (four slots
+// whatever the rows: bf16 -> fp8 500x512 5.8 us, now 3.1), one for copies
+// (4000x1024 4.7 us, 5.2 with two), any for fills, which wait for no load.
+SlotGrid slot_grid(int64_t rows, int64_t cols, int most_slots, int fill_blocks) {
   const int64_t slots = (cols + 7) / 8;
-  if (slots > tile::kThreads / 2) {
+  if (slots > most_slots) {
     const int64_t per_block = (int64_t)tile::kThreads * tile::kSlots * 8;
     return SlotGrid{dim3((unsigned)((cols + per_block - 1) / per_block),
-                         (unsigned)(rows < 65535 ? rows : 65535)), -1};
+                         (unsigned)(rows < 65535 ? rows : 65535)), -1, tile::kSlots};
   }
   const int tpr_log2 = ilog2(slots);
-  const int64_t per_block = (int64_t)(tile::kThreads >> tpr_log2) * tile::kSlots;
-  const int64_t blocks = (rows + per_block - 1) / per_block;
-  return SlotGrid{dim3((unsigned)(blocks < (1 << 20) ? blocks : 1 << 20)), tpr_log2};
+  const int64_t rpp = tile::kThreads >> tpr_log2;
+  int spt = tile::kSlots;
+  while (spt > 1 && rows < fill_blocks * rpp * spt) spt /= 2;
+  const int64_t blocks = (rows + rpp * spt - 1) / (rpp * spt);
+  return SlotGrid{dim3((unsigned)(blocks < (1 << 20) ? blocks : 1 << 20)), tpr_log2, spt};
 }
 
 template <Elt S, Elt D>
 hipError_t copy_typed(const CopyArgs& a, hipStream_t s) {
-  const SlotGrid g = slot_grid(a.rows, a.cols);
+  // Slots of 32 bytes: 65536x1024 f32 -> bf16 81 us shared, 69 a row each.
+  const bool words = EltInfo<S>::bytes == 4 || EltInfo<D>::bytes == 4;
+  const SlotGrid g = slot_grid(a.rows, a.cols, words ? 64 : 128, 512);
   auto kern = g.tpr_log2 < 0 ? copy_convert_kernel<S, D, true> : copy_convert_kernel<S, D, false>;
   hipLaunchKernelGGL(kern, g.grid, dim3(tile::kThreads), 0, s, a.src, a.ld_src,
-                     a.dst, a.ld_dst, a.rows, a.cols, g.tpr_log2);
+                     a.dst, a.ld_dst, a.rows, a.cols, g.tpr_log2, g.spt);
   return hipGetLastError();
 }
 
@@ -748,19 +770,19 @@ hipError_t copy_from(const CopyArgs& a, hipStream_t s) {
 
 template <int BYTES>
 hipError_t copy_raw(const CopyArgs& a, hipStream_t s) {
-  const SlotGrid g = slot_grid(a.rows, a.cols);
+  const SlotGrid g = slot_grid(a.rows, a.cols, BYTES >= 4 ? 64 : 128, 256);
   auto kern = g.tpr_log2 < 0 ? copy_raw_kernel<BYTES, true> : copy_raw_kernel<BYTES, false>;
   hipLaunchKernelGGL(kern, g.grid, dim3(tile::kThreads), 0, s, a.src, a.ld_src,
-                     a.dst, a.ld_dst, a.rows, a.cols, g.tpr_log2);
+                     a.dst, a.ld_dst, a.rows, a.cols, g.tpr_log2, g.spt);
   return hipGetLastError();
 }
 
 template <int BYTES>
 hipError_t fill_bytes(const FillArgs& a, hipStream_t s) {
-  const SlotGrid g = slot_grid(a.rows, a.cols);
+  const SlotGrid g = slot_grid(a.rows, a.cols, BYTES == 8 ? 64 : 128, 0);
   auto kern = g.tpr_log2 < 0 ? fill_kernel<BYTES, true> : fill_kernel<BYTES, false>;
   hipLaunchKernelGGL(kern, g.grid, dim3(tile::kThreads), 0, s, a.dst, a.ld, a.rows,
-                     a.cols, a.bits, g.tpr_log2);
+                     a.cols, a.bits, g.tpr_log2, g.spt);
   return hipGetLastError();
 }
 
