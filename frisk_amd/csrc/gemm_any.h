@@ -10,10 +10,11 @@
 //  * One BT x BT output tile per 256-thread workgroup (4 waves, 2x2, each a
 //    quarter of it as accumulators of the 32x32 MFMA), BT 128 or 64, K in
 //    stages of 128 bytes of LDS: the operand tiles, LDS swizzles and fragment
-//    reads of gemm_tile.h.  What bounds a stage is LDS traffic and its waits,
-//    0.70 us of a CU for a 128 tile and 0.28 us for a 64 tile whatever the
-//    depth of the loads, so BT and the K slices follow from the whole rounds
-//    of tiles over the CUs (plan::any_plan).
+//    reads of gemm_tile.h.  What bounds a stage is LDS traffic and its waits:
+//    1.1 us for a 128 tile alone on its CU (1111x3333x1777 f16, 28 stages in
+//    34 us), 0.8 in many rounds of two per CU (3824x8704x2225), 0.3 to 0.4
+//    for a 64 tile.  BT and the K slices follow from the rounds of tiles over
+//    the CUs (plan::any_plan).
 //  * LDS-DMA needs aligned pieces, so a stage goes through registers: each
 //    lane loads 16 bytes from an element-aligned address (a global load takes
 //    any alignment) and writes them where the DMA would have put them, halfway

@@ -173,17 +173,33 @@ inline SplitPlan split_plan(const GemmShape& g, int cus) {
 // The any-alignment kernel (gemm_any.h): 128x128 tiles (big) or 64x64, K
 // slices on stage boundaries (128 bytes), 32-bit partials of every type pair
 // in rows of any_partial_pitch elements, summed by a second launch.  The
-// choice with the least estimated time: whole rounds of tiles over the CUs at
-// the time a stage takes a CU (us, measured: 0.70 and 0.28; f32, whose MFMA
-// is 16 times slower, 1.9 and 0.48), and for a split the partials' traffic and
-// about 5 us of second launch and scratch (9x897x528: 8.0 us unsplit, 12.6
-// split).  Measured, us, over tiles and slices: 1111x3333x1777 f16 35.5 on
-// 128 tiles, 45.5 on 64; 33x189x896 16.9 and 9.1; 1589x256x13953 fp8 172 and
-// 75; 2x210x13418 153 and 64 unsplit, 13.8 and 12.4 in 32 slices.  The
-// partials stay within the scratch of frisk_gemm_noalloc.
+// choice with the least estimated time: a launch (3.2 us), the stages at the
+// time one takes a CU, alone or times the rounds of tiles over the CUs, the
+// tiles' epilogues, and for a split the partials' traffic and a second launch.
+// The constants are fitted to 1100 timings (38 shapes, f16, f32, int8, fp8,
+// both tiles, 1 .. 64 slices, operands from HBM), within 11% rms, e.g. us
+// measured and estimated: 1111x3333x1777 f16 128 tiles 34.2 and 25.6, 64 tiles
+// 45.1 and 35.8; 1500x1500x5001 72.7 and 63.9, in 3 slices 54.7 and 54.7;
+// 33x189x897 9.4 and 8.2; 2x210x13419 in 12 slices 11.6 and 12.8.  The choice is
+// within 0.5% of the fastest on average, 25% at worst.  The partials stay within
+// the scratch of frisk_gemm_noalloc.
 // ---------------------------------------------------------------------------
 inline int64_t any_partial_pitch(int64_t n) { return (n + 3) & ~(int64_t)3; }
 constexpr int64_t kAnyMaxPartial = 64ll << 20;
+
+// us of a stage on a CU: [64 tiles, 128 tiles][one workgroup per CU, a round
+// of several].
+struct AnyStage {
+  double us[2][2];
+};
+inline AnyStage any_stage(int in) {
+  switch (in) {
+    case kF32: return {{{0.65, 0.60}, {2.37, 2.11}}};  // (a matrix rate 16 times lower)
+    case kI8: return {{{0.31, 0.40}, {0.93, 0.83}}};
+    case kE4M3: return {{{0.27, 0.25}, {0.71, 0.55}}};  // (half the K of the others)
+    default: return {{{0.29, 0.27}, {0.75, 0.67}}};
+  }
+}
 
 inline SplitPlan any_plan(const GemmShape& g, int cus, bool workspace) {
   const int64_t kb = g.k * dtype_bytes(g.in);
@@ -195,15 +211,19 @@ inline SplitPlan any_plan(const GemmShape& g, int cus, bool workspace) {
   double best_us = -1.0;
   for (const int64_t bt : {64, 128}) {
     const int64_t tiles = ((g.m + bt - 1) / bt) * ((g.n + bt - 1) / bt);
-    const double stage_us = g.in == kF32 ? (bt == 64 ? 0.48 : 1.9) : bt == 64 ? 0.28 : 0.70;
+    if (tiles * 256 > UINT32_MAX) continue;  // threads of a grid
+    const AnyStage st = any_stage(g.in);
     // (Few candidates: the plan is made on every call.)
     for (const int64_t sl : {1, 2, 3, 4, 6, 8, 12, 16, 24, 32, 48, 64}) {
       if (sl > std::max<int64_t>(most, 1)) break;
       const int64_t kb_slice = sl == 1 ? kb : (chunks + sl - 1) / sl * 128;
       const int64_t slices = (kb + kb_slice - 1) / kb_slice;
       if (slices < sl) continue;
-      const double us = rounds(tiles * slices, cus) * (double)((kb_slice + stage - 1) / stage) * stage_us +
-                        (slices > 1 ? 5.0 + (double)slices * slice_bytes * 2 / (kPartialBw * 1e-6) : 0.0);
+      const double r = rounds(tiles * slices, cus);
+      const double us = 3.2 + r * (bt == 128 ? 1.4 : 0.6) +
+                        (double)((kb_slice + stage - 1) / stage) *
+                            (r <= 1 ? st.us[bt == 128][0] : r * st.us[bt == 128][1]) +
+                        (slices > 1 ? 3.8 + (double)slices * slice_bytes * 2 / 6.2e6 : 0.0);
       if (best_us >= 0 && us >= best_us) continue;
       best_us = us;
       best = SplitPlan{(int)slices, kb_slice, slices > 1 ? slices * slice_bytes : 0, bt == 128};
