@@ -24,9 +24,11 @@ PAIRS = [(torch.bfloat16, torch.bfloat16), (torch.bfloat16, torch.float32),
          (FP8, torch.bfloat16), (FP8, torch.float16), (FP8, torch.float32),
          (torch.int8, torch.int32), (torch.float32, torch.float32)]
 TOL = {torch.bfloat16: 1e-2, torch.float16: 1e-2, torch.float32: 1e-5}
-# One element, a matrix under 16 bytes, a K inside one piece, the edges of the
-# 128x128 tile and of the 128-byte stage (128, 64 and 32 elements), one past
-# them, and a K that splits (16 stages and more) with a partial last slice.
+# One element, a matrix under 16 bytes, a K inside one piece, the edges of two
+# 64x64 tiles (which the plan takes for all of these; 128x128:
+# test_gemm_any_tiles_gpu.py) and of the 128-byte stage (128, 64 and 32
+# elements), one past them, and a K that splits (16 stages and more) with a
+# partial last slice.
 SHAPES = [(1, 1, 1), (2, 3, 3), (5, 7, 9), (1, 129, 31), (33, 1, 127), (127, 130, 129),
           (128, 128, 128), (129, 255, 65), (3, 70, 2100), (130, 5, 4109)]
 

@@ -16,8 +16,9 @@ pytestmark = pytest.mark.gpu
 # sixteen, with a partial last chunk and runs of no chunk.
 ROWS = [(2100, 1500), (600, 2049), (3, 16385), (40, 28653), (1, 70001)]
 # Axis 0: under 256 rows (one, a few and 32 runs of eight), two passes (partial
-# last block; one block; narrow with many blocks), one pass of 1024 threads
-# (12800 columns), and a run of more than 256 rows.
+# last block; one block; narrow with many blocks, whose longest run without a
+# workspace is 256 rows; strips that leave part of a round empty), and the same
+# in one pass of 1024 threads.  (Longer runs: test_reduce_deep_gpu.py.)
 COLS = [(1, 900), (26, 1433), (112, 1587), (255, 70), (256, 515), (449, 665), (17921, 9),
         (600, 12801), (3000, 12805)]
 
