@@ -3,7 +3,7 @@
 // runs with.  Host-only C++ without HIP, so that two consumers share one
 // decision: the C-ABI (capi.hip, gemm.hip, the launchers) follows it for
 // every call that names no variant, and the layout target of the IR
-// (frisk_amd/ir: F.frisk.gemm_launch_plan / attn_launch_plan) reports it as
+// (frisk_amd/ir: F.frisk.gemm_launch_plan / attention_launch_plan) reports it as
 // the launch contract of a whole-matrix GEMM or an attention program, which
 // execute() then requests explicitly.  The reference makes the matching
 // decision at compile time, in its SM90 layout target's MMA binding
