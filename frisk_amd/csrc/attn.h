@@ -641,7 +641,7 @@ static hipError_t launch_fewq(const AttnArgs& a, hipStream_t stream);
 template <Elt T, Elt OUT, int D, bool CAUSAL>
 static hipError_t launch_attn(const AttnArgs& a, hipStream_t stream) {
   const plan::AttnLaunch L =
-      plan::attn_launch(a.batch * a.heads, a.seq_q, a.seq_k, D, CAUSAL, device_cus(), a.waves);
+      plan::attn_launch(a.batch * a.heads, a.seq_q, a.seq_k, D, a.k_dmajor != 0, CAUSAL, device_cus(), a.waves);
   if (L.few)
     return a.k_dmajor ? launch_fewq<T, OUT, D, CAUSAL, true>(a, stream)
                       : launch_fewq<T, OUT, D, CAUSAL, false>(a, stream);

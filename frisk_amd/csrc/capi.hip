@@ -499,7 +499,7 @@ int check_attn(const frisk_attn_desc* d, bool ptrs, frisk::AttnArgs& a) {
 }
 
 int64_t attn_workspace(const frisk::AttnArgs& a) {
-  return frisk::plan::attn_workspace(a.batch * a.heads, a.seq_q, a.seq_k, a.head_dim,
+  return frisk::plan::attn_workspace(a.batch * a.heads, a.seq_q, a.seq_k, a.head_dim, a.k_dmajor != 0,
                                      frisk::device_cus());
 }
 

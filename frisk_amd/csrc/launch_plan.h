@@ -555,14 +555,17 @@ inline int attn_waves(int64_t batch_heads, int64_t seq_q, int64_t head_dim, bool
 //   d 16   128 keys 1.16 1.16 2.01 2.75    256 0.92 0.99 1.51 1.80   768 0.61 0.66 0.89 0.97
 //   d 64   128 keys 1.04 1.07 1.49 1.76    256 0.83 0.96 1.17 1.43   768 0.56 0.74 0.90  -
 //   d 128   64 keys 1.15 1.02 1.45 1.74    128 0.95 0.98 1.28 1.39   512 0.67 0.86 0.92  -
+// (d 128 with K stored transposed, 300 heads, 2 and 32 queries: 512 keys 1.05
+// and 1.18, 4096 1.07 and 1.07; one round of heads gains as the others do.)
 constexpr int64_t kFewQ = 32;
 constexpr int few_waves(int64_t head_dim) { return head_dim == 128 ? 4 : head_dim == 64 ? 8 : 16; }
 
-inline bool attn_few(int64_t batch_heads, int64_t seq_q, int64_t seq_k, int64_t head_dim, int cus) {
+inline bool attn_few(int64_t batch_heads, int64_t seq_q, int64_t seq_k, int64_t head_dim, bool k_transposed,
+                     int cus) {
   const int64_t nkb = (seq_k + 63) / 64;
   if (seq_q > kFewQ || batch_heads * 64 * few_waves(head_dim) > UINT32_MAX) return false;  // (threads of a grid)
   if (batch_heads <= cus) return nkb >= (head_dim == 128 ? 2 : head_dim == 64 ? 3 : 4);
-  return nkb >= (head_dim == 128 ? 7 : 12);
+  return head_dim == 128 ? nkb >= 7 && !k_transposed : nkb >= 12;
 }
 
 // The kernel and waves per workgroup of a call; `waves` (4, 8 or 0) chooses
@@ -572,8 +575,8 @@ struct AttnLaunch {
   int waves;
 };
 inline AttnLaunch attn_launch(int64_t batch_heads, int64_t seq_q, int64_t seq_k, int64_t head_dim,
-                              bool causal, int cus, int waves) {
-  if (attn_few(batch_heads, seq_q, seq_k, head_dim, cus)) return AttnLaunch{true, few_waves(head_dim)};
+                              bool k_transposed, bool causal, int cus, int waves) {
+  if (attn_few(batch_heads, seq_q, seq_k, head_dim, k_transposed, cus)) return AttnLaunch{true, few_waves(head_dim)};
   return AttnLaunch{false, waves ? waves : attn_waves(batch_heads, seq_q, head_dim, causal, cus)};
 }
 
@@ -607,8 +610,8 @@ inline int attn_splits(int64_t batch_heads, int64_t seq_q, int64_t seq_k, int64_
   return best;
 }
 inline int64_t attn_workspace(int64_t batch_heads, int64_t seq_q, int64_t seq_k, int64_t head_dim,
-                              int cus) {
-  if (!attn_few(batch_heads, seq_q, seq_k, head_dim, cus)) return 0;
+                              bool k_transposed, int cus) {
+  if (!attn_few(batch_heads, seq_q, seq_k, head_dim, k_transposed, cus)) return 0;
   const int64_t s = attn_splits(batch_heads, seq_q, seq_k, head_dim, cus);
   return s > 1 ? batch_heads * s * seq_q * (head_dim + 2) * 4 : 0;
 }

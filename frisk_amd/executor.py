@@ -678,7 +678,8 @@ def execute(module, kernel: str, tensors: Sequence, *, stream=None, causal: bool
     # A K stored [B, H, D, S] (the reference's FA tile program) is read in
     # place by the kernel's transposed-K variant; the waves per workgroup
     # come from the attention launch contract.
-    L = fr.attention_launch_plan(p.batch * p.heads, p.seq, p.head_dim, causal, _device_cus())
+    L = fr.attention_launch_plan(p.batch * p.heads, p.seq, p.head_dim, causal, _device_cus(),
+                                 k_transposed=p.k_transposed)
     p.waves = {"causal" if causal else "full": L["waves"]}
     return rt.attn_fwd(q, kk, v, o, causal=causal, sm_scale=sm_scale, stream=stream,
                        k_transposed=p.k_transposed, waves=rt.requested_waves(L))

@@ -1295,15 +1295,15 @@ void bindFrisk(py::module_& m) {
      py::arg("trans_a") = false, py::arg("trans_b") = false, py::arg("cus") = 256,
      py::arg("workspace") = true, py::arg("matrix_cores") = true);
   m.def("attention_launch_plan", [](int64_t batchHeads, int64_t seqQ, int64_t headDim, bool causal,
-                                    int64_t cus, std::optional<int64_t> seqK) {
+                                    int64_t cus, std::optional<int64_t> seqK, bool kTransposed) {
     const AttentionLaunchContract c =
-        cdna4AttentionLaunch(batchHeads, seqQ, seqK.value_or(seqQ), headDim, causal, cus);
+        cdna4AttentionLaunch(batchHeads, seqQ, seqK.value_or(seqQ), headDim, kTransposed, causal, cus);
     py::dict d;
     d["kernel"] = c.kernel;
     d["waves"] = c.waves;
     return d;
   }, py::arg("batch_heads"), py::arg("seq_q"), py::arg("head_dim"), py::arg("causal") = false,
-     py::arg("cus") = 256, py::arg("seq_k") = py::none());
+     py::arg("cus") = 256, py::arg("seq_k") = py::none(), py::arg("k_transposed") = false);
   m.def("cost_profile_defaults", []() {
     CostProfile p = CostProfile::defaults();
     py::dict d;

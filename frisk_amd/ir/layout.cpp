@@ -317,13 +317,14 @@ GemmLaunchContract cdna4GemmLaunch(int64_t m, int64_t n, int64_t k, Type in, Typ
 }
 
 AttentionLaunchContract cdna4AttentionLaunch(int64_t batchHeads, int64_t seqQ, int64_t seqK,
-                                             int64_t headDim, bool causal, int64_t cus) {
+                                             int64_t headDim, bool kTransposed, bool causal,
+                                             int64_t cus) {
   if (batchHeads <= 0 || seqQ <= 0 || seqK <= 0)
     throw InvalidArgument("launch contract: sizes must be positive");
   if (headDim != 16 && headDim != 32 && headDim != 64 && headDim != 128)
     throw InvalidArgument("launch contract: the attention kernel takes head_dim 16, 32, 64 or 128");
   const frisk::plan::AttnLaunch L =
-      frisk::plan::attn_launch(batchHeads, seqQ, seqK, headDim, causal, (int)cus, 0);
+      frisk::plan::attn_launch(batchHeads, seqQ, seqK, headDim, kTransposed, causal, (int)cus, 0);
   return AttentionLaunchContract{L.few ? "attn_fewq" : "attn_fwd", L.waves};
 }
 

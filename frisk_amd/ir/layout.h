@@ -135,6 +135,7 @@ struct AttentionLaunchContract {
   int64_t waves = 0;
 };
 AttentionLaunchContract cdna4AttentionLaunch(int64_t batchHeads, int64_t seqQ, int64_t seqK,
-                                             int64_t headDim, bool causal, int64_t cus);
+                                             int64_t headDim, bool kTransposed, bool causal,
+                                             int64_t cus);
 
 }  // namespace fir

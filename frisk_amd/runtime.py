@@ -375,7 +375,8 @@ def attn_fwd(q, k, v, o, *, causal=False, sm_scale=None, lse=None, stream=None,
     """O = softmax(sm_scale . Q K^T [causal mask]) V on the GPU.  K is
     [batch, heads, seq_k, head_dim], or [batch, heads, head_dim, seq_k] with
     k_transposed=True (read in place).  `waves` (4 or 8) requests the
-    workgroup shape; 0 lets the library choose."""
+    workgroup shape; 0 lets the library choose.  Few queries over many keys
+    take scratch from torch's caching allocator, on the call's stream."""
     d = attn_desc(q, k, v, o, causal=causal, sm_scale=sm_scale, lse=lse, k_transposed=k_transposed,
                   waves=waves)
     lib, ws, need = load(), None, 0

@@ -217,8 +217,8 @@ typedef struct frisk_attn_desc {
   /* Waves per workgroup (32 queries each): 0, the library chooses (the
    * launch contract layout inference gives an attention program); 4 or 8
    * (8 needs head_dim 128).  A call that the few-query kernel takes (up to
-   * 32 queries and more than 64 to 704 keys, by head_dim and the number of
-   * heads; "attn_fewq" in the launch contract), whose 4, 8 or 16 waves divide
+   * 32 queries and more than 64 to 704 keys, by head_dim, the number of heads
+   * and K's storage; "attn_fewq" in the launch contract), whose 4, 8 or 16 waves divide
    * the keys, is checked for it and runs the same with any.  The result bits
    * do not depend on it. */
   int32_t waves;

@@ -16,17 +16,18 @@ CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))),
 def few(tmp_path_factory):
     """plan::attn_few on 256 CUs for (heads, queries, keys, head_dim) tuples."""
     d = tmp_path_factory.mktemp("plan")
-    src, exe = d / "plan.cpp", d / "plan"
+    src = d / "plan.cpp"
     src.write_text(f"""#include "{CSRC}/launch_plan.h"
 #include <cstdio>
 #include <cstdlib>
 int main(int n, char** v) {{
   for (int i = 1; i + 3 < n; i += 4)
-    printf("%d ", frisk::plan::attn_few(atoll(v[i]), atoll(v[i + 1]), atoll(v[i + 2]), atoll(v[i + 3]), 256));
+    printf("%d ", frisk::plan::attn_few(atoll(v[i]), atoll(v[i + 1]), atoll(v[i + 2]), atoll(v[i + 3]), KT, 256));
 }}""")
-    subprocess.run(["g++", "-std=c++17", str(src), "-o", str(exe)], check=True)
-    return lambda calls: [x == "1" for x in subprocess.run(
-        [str(exe), *(str(x) for c in calls for x in c)], check=True, capture_output=True,
+    for kt in (0, 1):
+        subprocess.run(["g++", "-std=c++17", f"-DKT={kt}", str(src), "-o", str(d / f"plan{kt}")], check=True)
+    return lambda calls, kt=False: [x == "1" for x in subprocess.run(
+        [str(d / f"plan{int(kt)}"), *(str(x) for c in calls for x in c)], check=True, capture_output=True,
         text=True).stdout.split()]
 
 
@@ -40,6 +41,13 @@ def test_few_queries_need_enough_keys_for_their_heads(few, d, waves):
     # A grid of workgroups holds fewer than 2^32 threads.
     most = (1 << 32) // (64 * waves)
     assert few([(most - 1, 1, 4096, d), (most, 1, 4096, d)]) == [True, False]
+
+
+def test_transposed_keys_at_head_dim_128_in_one_round_of_heads(few):
+    calls = [(256, 2, 4096, 128), (257, 2, 4096, 128), (1024, 32, 512, 128), (257, 2, 4096, 64)]
+    assert few(calls) == [True] * 4 and few(calls, kt=True) == [True, False, False, True]
+    plans = [F.frisk.attention_launch_plan(b, q, d, seq_k=k, k_transposed=True)["kernel"] for b, q, k, d in calls]
+    assert plans == ["attn_fewq", "attn_fwd", "attn_fwd", "attn_fewq"]
 
 
 def contract(bh, sq, sk, d):
